@@ -2,10 +2,10 @@
 //
 // Per layer the reference runs q_norm, k_norm, two permutes, mylib::rope and
 // mylib::update_kv_padded (aspire/models/sparse_draft_transformer.py:149-171):
-// six launches and four round trips of q / k through HBM. Here one wave
-// handles one head of one token (lane i owns rotated pair i, i.e. dims 2i and
-// 2i+1 after the permute): it normalises, rotates and writes q in place and
-// k / v into the page pool at the token's append position.
+// six launches and four round trips of q / k through HBM. Here a few waves
+// take a token: 16 lanes own a head (lane j its rotated pairs 4j .. 4j + 3,
+// dims 8j .. 8j + 7 after the permute), normalise and rotate it, write q in
+// place and k / v into the page pool at the token's append position.
 //
 //   * RMSNorm (transformer.py:505-516): fp32 sum of squares (wave sum),
 //     x * (1 / sqrt(mean + eps)) rounded to bf16, times the bf16 weight,
@@ -17,7 +17,6 @@
 //     frequencies once, including the Llama 3.1 smoothing), accurate sincosf,
 //     (a, b) -> (a cos - b sin, b cos + a sin) in fp32, rounded to bf16;
 //   * append: the row / slot rule of the plain append (append_locate).
-#include <algorithm>
 #include <cmath>
 
 #include "common.h"
@@ -53,65 +52,176 @@ struct RopeParams {
   int32_t write_k;
 };
 
-__device__ __forceinline__ float bf16_to_f(uint16_t h) { return __uint_as_float(uint32_t(h) << 16); }
-__device__ __forceinline__ uint16_t f_to_bf16(float f) { return static_cast<uint16_t>(bf16_rne_bits(f)); }
+// Head slots of one wave pass: 4 groups of 16 lanes, one head each.
+constexpr int kRopeHeads = 4;
+constexpr int kRopeWaves = 4;   // waves per workgroup
 
-constexpr int kHeadsPerBlock = 4;  // one wave per head
+__device__ __forceinline__ float lo_bf(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float hi_bf(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-// Grid (tokens, ceil((hq + hkv) / 4)): wave w of block (tok, hb) prepares
-// head 4 * hb + w of token tok (q heads first, then k heads) and, when
-// 4 * hb + w < hkv, copies that v head into the page.
-__global__ __launch_bounds__(256) void qk_norm_rope_append_kernel(RopeParams p) {
-  const int tok = blockIdx.x;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int h = blockIdx.y * kHeadsPerBlock + wave;
-  // rope position: row b of indptr owns tok (last b with indptr[b] <= tok < indptr[b + 1])
-  int pos = -1;
-  {
-    const int b = wave_last_le(p.indptr, p.num_rows, tok);
-    if (b >= 0 && tok < p.indptr[b + 1]) pos = p.offsets[b] + tok - p.indptr[b];
+// Sum over the 16 lanes of each DPP row.
+__device__ __forceinline__ float row_sum_f(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));
+  return v;
+}
+
+// The 8 inputs of lane j of a head as 4 words: pairs 4j .. 4j + 3 are dims (4j + e, 64 + 4j + e)
+// with the permute (words 0-1: the first halves, 2-3: the second), (8j + 2e, 8j + 2e + 1) without.
+template <bool kWide>
+__device__ __forceinline__ uint4 load_lane_dims(const uint16_t* row, int j, bool permute) {
+  const int d0 = permute ? 4 * j : 8 * j, d1 = permute ? kPairs + 4 * j : 8 * j + 4;
+  if (kWide) {
+    const uint2 x = *reinterpret_cast<const uint2*>(row + d0), y = *reinterpret_cast<const uint2*>(row + d1);
+    return make_uint4(x.x, x.y, y.x, y.y);
   }
-  pos = wave_uniform(pos);
-  int entry = -1, slot = 0;
-  const bool append = p.cache != nullptr &&
-                      append_locate(p.indptr, p.num_seq, p.page_indptr, p.last_page_len, p.page_size, tok, entry, slot);
-  uint16_t* page_k = nullptr;
-  if (append) page_k = p.cache + int64_t(p.page_indices[entry]) * p.c_sp + int64_t(slot) * p.c_st;
+  auto word = [&](int d) { return uint32_t(row[d]) | (uint32_t(row[d + 1]) << 16); };
+  return make_uint4(word(d0), word(d0 + 2), word(d1), word(d1 + 2));
+}
+__device__ __forceinline__ void split_pairs(const uint4& w, bool permute, float* a, float* b) {
+  if (permute) {
+    a[0] = lo_bf(w.x), a[1] = hi_bf(w.x), a[2] = lo_bf(w.y), a[3] = hi_bf(w.y);
+    b[0] = lo_bf(w.z), b[1] = hi_bf(w.z), b[2] = lo_bf(w.w), b[3] = hi_bf(w.w);
+  } else {
+    a[0] = lo_bf(w.x), a[1] = lo_bf(w.y), a[2] = lo_bf(w.z), a[3] = lo_bf(w.w);
+    b[0] = hi_bf(w.x), b[1] = hi_bf(w.y), b[2] = hi_bf(w.z), b[3] = hi_bf(w.w);
+  }
+}
+__device__ __forceinline__ void round_pair(float& x, float& y) {
+  const uint32_t w = pack_bf16x2_rne(x, y);
+  x = lo_bf(w);
+  y = hi_bf(w);
+}
 
-  if (h < p.hq + p.hkv) {
+// wpt consecutive waves share a token; wave `part` of them takes head quads part, part + wpt, ...
+// of the token's q heads, k heads and (when appending) v heads, in that order. A head is read
+// with 8-byte and written with 16-byte accesses (kWide: q, k and the weights allow them), and a
+// wave computes the token's 64 angles once, one per lane, handing every lane its four through the
+// wave's LDS slice. Bound by HBM at prompt-chunk sizes, by the chain of loads (row search, row
+// metadata, page id) plus one sincosf at decode sizes. One wave per (token, head) with 2-byte
+// loads, two searches and a sincosf for every head took 168 us for 8,192 tokens of 32 q / 8 kv
+// heads (1.2 TB/s, bound by the sincosf and address arithmetic) where this takes 48 us (4.2 TB/s);
+// 208 tokens 6.3 -> 4.8 us.
+template <bool kWide>
+__global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(RopeParams p, int total_tokens, int wpt_log2) {
+  __shared__ float2 rot[kRopeWaves][kPairs];
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_uniform(threadIdx.x >> 6);
+  const int unit = blockIdx.x * kRopeWaves + wave;
+  const int tok = unit >> wpt_log2;
+  const int part = unit & ((1 << wpt_log2) - 1);
+  if (tok >= total_tokens) return;
+  const int j = lane & 15, grp = lane >> 4;
+  const bool permute = p.permute != 0, norm = p.q_w != nullptr;
+  const int n_qk = p.hq + p.hkv;
+  const int n_all = p.cache != nullptr && p.v != nullptr ? n_qk + p.hkv : n_qk;
+  const int step = kRopeHeads << wpt_log2;
+
+  // a head's words: q / k dims for the rotation, 16 bytes of v for the copy
+  auto load = [&](int h) -> uint4 {
+    uint4 w = make_uint4(0, 0, 0, 0);
+    if (h < p.hq) {
+      w = load_lane_dims<kWide>(p.q + int64_t(tok) * p.q_st + int64_t(h) * p.q_sh, j, permute);
+    } else if (h < n_qk) {
+      w = load_lane_dims<kWide>(p.k + int64_t(tok) * p.k_st + int64_t(h - p.hq) * p.k_sh, j, permute);
+    } else if (h < n_all) {
+      w = *reinterpret_cast<const uint4*>(p.v + int64_t(tok) * p.v_st + int64_t(h - n_qk) * p.v_sh + 8 * j);
+    }
+    return w;
+  };
+  // the first quad's loads and the weights are requested before the position look-up they do not need
+  int h = part * kRopeHeads + grp;
+  uint4 cur = load(h);
+  uint4 qw = make_uint4(0, 0, 0, 0), kw = qw;
+  if (norm) {
+    qw = load_lane_dims<kWide>(p.q_w, j, permute);
+    kw = load_lane_dims<kWide>(p.k_w, j, permute);
+  }
+
+  // one search serves both positions: the row b that owns the token (last b with indptr[b] <= tok),
+  // and the append's rows are its first num_seq
+  int pos = -1;
+  uint16_t* page_k = nullptr;
+  const int b = wave_last_le(p.indptr, p.num_rows, tok);
+  if (b >= 0) {
+    const int begin = p.indptr[b], end = p.indptr[b + 1];
+    if (tok < end) {
+      pos = wave_uniform(p.offsets[b] + tok - begin);
+      if (p.cache != nullptr && b < p.num_seq) {
+        const int first = p.page_indptr[b];
+        const int pages = p.page_indptr[b + 1] - first;
+        const int seq_len = max(pages - 1, 0) * p.page_size + p.last_page_len[b];
+        const int ps = tok + seq_len - end;
+        if (pages != 0 && ps >= 0 && ps < (pages - 1) * p.page_size + p.last_page_len[b])
+          page_k = p.cache + int64_t(p.page_indices[first + ps / p.page_size]) * p.c_sp +
+                   int64_t(ps % p.page_size) * p.c_st;
+      }
+    }
+  }
+
+  {
     float c = 1.f, s = 0.f;
     if (pos >= 0) sincosf(static_cast<float>(pos) * p.freq[lane], &s, &c);
-    const int in0 = p.permute ? lane : 2 * lane;
-    const int in1 = p.permute ? lane + kPairs : 2 * lane + 1;
-    const bool is_q = h < p.hq;
-    uint16_t* row = is_q ? p.q + int64_t(tok) * p.q_st + int64_t(h) * p.q_sh
-                         : p.k + int64_t(tok) * p.k_st + int64_t(h - p.hq) * p.k_sh;
-    float x0 = bf16_to_f(row[in0]);
-    float x1 = bf16_to_f(row[in1]);
-    const uint16_t* w = is_q ? p.q_w : p.k_w;
-    if (w != nullptr) {
-      const float ms = wave_sum_f(x0 * x0 + x1 * x1) / float(kHeadDim);
-      const float r = 1.f / sqrtf(ms + p.eps);
-      x0 = bf16_to_f(f_to_bf16(bf16_to_f(f_to_bf16(x0 * r)) * bf16_to_f(w[in0])));
-      x1 = bf16_to_f(f_to_bf16(bf16_to_f(f_to_bf16(x1 * r)) * bf16_to_f(w[in1])));
-    }
-    float y0 = x0, y1 = x1;
-    if (pos >= 0) {
-      y0 = x0 * c - x1 * s;
-      y1 = x1 * c + x0 * s;
-    }
-    const uint32_t packed = uint32_t(f_to_bf16(y0)) | (uint32_t(f_to_bf16(y1)) << 16);
-    // every lane has read its inputs before any lane stores (one wave per head)
-    if (is_q || p.write_k) *reinterpret_cast<uint32_t*>(row + 2 * lane) = packed;
-    if (!is_q && append)
-      *reinterpret_cast<uint32_t*>(page_k + int64_t(h - p.hq) * p.c_sh + 2 * lane) = packed;
+    rot[wave][lane] = make_float2(c, s);
   }
-  if (append && p.v != nullptr && h < p.hkv && lane < kHeadDim / 8) {
-    uint16_t* page_v = page_k + p.c_skv;
-    const uint16_t* src = p.v + int64_t(tok) * p.v_st;
-    *reinterpret_cast<uint4*>(page_v + int64_t(h) * p.c_sh + lane * 8) =
-        *reinterpret_cast<const uint4*>(src + int64_t(h) * p.v_sh + lane * 8);
+  float c[4], s[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float2 r = rot[wave][4 * j + e];
+    c[e] = r.x;
+    s[e] = r.y;
+  }
+
+  for (; wave_uniform(h - grp) < n_all; h += step) {
+    const uint4 next = load(h + step);  // heads past the last one load nothing
+    const uint4 w = cur;
+    cur = next;
+    if (h >= n_qk) {
+      if (h < n_all && page_k != nullptr)
+        *reinterpret_cast<uint4*>(page_k + p.c_skv + int64_t(h - n_qk) * p.c_sh + 8 * j) = w;
+      continue;
+    }
+    const bool is_q = h < p.hq;
+    float x[4], y[4];
+    split_pairs(w, permute, x, y);
+    if (norm) {
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss += x[e] * x[e] + y[e] * y[e];
+      const float r = 1.f / sqrtf(row_sum_f(ss) / float(kHeadDim) + p.eps);
+      float wx[4], wy[4];
+      split_pairs(is_q ? qw : kw, permute, wx, wy);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] *= r;
+        y[e] *= r;
+        round_pair(x[e], y[e]);
+        x[e] *= wx[e];
+        y[e] *= wy[e];
+        round_pair(x[e], y[e]);
+      }
+    }
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] = pos >= 0 ? pack_bf16x2_rne(x[e] * c[e] - y[e] * s[e], y[e] * c[e] + x[e] * s[e])
+                      : pack_bf16x2_rne(x[e], y[e]);
+    }
+    // every lane of the wave has read its inputs before any lane stores
+    if (is_q || p.write_k) {
+      uint16_t* row = is_q ? p.q + int64_t(tok) * p.q_st + int64_t(h) * p.q_sh
+                           : p.k + int64_t(tok) * p.k_st + int64_t(h - p.hq) * p.k_sh;
+      if (kWide) {
+        *reinterpret_cast<uint4*>(row + 8 * j) = make_uint4(o[0], o[1], o[2], o[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(row + 8 * j + 2 * e) = o[e];
+      }
+    }
+    if (!is_q && page_k != nullptr)
+      *reinterpret_cast<uint4*>(page_k + int64_t(h - p.hq) * p.c_sh + 8 * j) = make_uint4(o[0], o[1], o[2], o[3]);
   }
 }
 
@@ -202,10 +312,19 @@ extern "C" int aspire_qk_norm_rope_append(const aspire_rope_args* a, void* strea
     ASPIRE_CHECK_ARG(a->v == nullptr || (aligned(a->v, 16) && a->v_stride_t % 8 == 0 && a->v_stride_h % 8 == 0),
                      "v rows must be 16-byte aligned");
   }
-  const int head_blocks = (std::max(a->num_qo_heads + a->num_kv_heads, a->num_kv_heads) + kHeadsPerBlock - 1) /
-                          kHeadsPerBlock;
-  hipLaunchKernelGGL(qk_norm_rope_append_kernel, dim3(a->total_tokens, head_blocks), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), p);
+  const bool wide = aligned(a->q, 16) && aligned(a->k, 16) && aligned(p.q_w, 8) && aligned(p.k_w, 8) &&
+                    a->q_stride_t % 8 == 0 && a->q_stride_h % 8 == 0 && a->k_stride_t % 8 == 0 &&
+                    a->k_stride_h % 8 == 0;
+  // Waves per token: enough waves to hide the look-up's latency, then as few as share one sincosf.
+  // us at 16 / 8 / 4 waves (32 q / 8 kv heads): 1 token 3.4 / 4.0 / 4.6, 16: 3.5 / 4.1 / 4.8, 80:
+  // 3.9 / 4.3 / 4.9, 208: 5.0 / 4.8 / 5.2, 512: 7.9 / 7.0 / 6.4, 8,192: 81 / 62 / 48; with 16 / 8
+  // heads 80: 3.9 / 3.6 / 4.2, 304: 5.5 / 4.4 / 4.7, 512: 7.7 / 5.1 / 5.1.
+  const int wpt_log2 = a->total_tokens <= 32 ? 4 : a->total_tokens <= 256 ? 3 : 2;
+  const int64_t units = int64_t(a->total_tokens) << wpt_log2;
+  const dim3 grid(unsigned((units + kRopeWaves - 1) / kRopeWaves));
+  const auto kernel = wide ? qk_norm_rope_append_kernel<true> : qk_norm_rope_append_kernel<false>;
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * kRopeWaves), 0, static_cast<hipStream_t>(stream), p, a->total_tokens,
+                     wpt_log2);
   ASPIRE_CHECK_LAUNCH();
   return ASPIRE_OK;
 }

@@ -77,3 +77,61 @@ def test_fused_norm_rope_append_config1_shape(gpu):
     assert torch.equal(got[:, 1], ref_cache[:, 1])       # V: exact copy
     bf16_close(got[:, 0][changed[:, 0]], ref_cache[:, 0][changed[:, 0]])
     assert torch.equal(kd.cpu(), k)                       # k itself is not rewritten by the fused op
+
+
+def pairs_close(got: torch.Tensor, ref: torch.Tensor):
+    """Rotated pairs against the oracle. The fp32 sums of the norm may be taken in another order, which
+    now and then moves one of a pair's two inputs by one bf16 step, at most 2^-7 of it, at each of its
+    two roundings; the rotation passes that on in full, so an output may be off by 2 * 2^-7 of the pair's
+    length (the rotation keeps it) besides its own step. All but a few are within their own step."""
+    g, r = got.double().cpu(), ref.double().cpu()
+    step = r.abs() * 2.0 ** -7 + 1e-6
+    length = torch.sqrt((r * r).unflatten(-1, (-1, 2)).sum(dim=-1, keepdim=True)).expand(*r.shape[:-1], -1, 2).flatten(-2)
+    off = (g - r).abs()
+    assert not (off > step + 2 * 2.0 ** -7 * length).any()
+    assert (off > step).double().mean().item() < 1e-4
+
+
+@pytest.mark.parametrize("hq,hkv,lens,width", [
+    (32, 8, [1], 128),                       # the smallest call: 16 waves a token
+    (7, 3, [5, 0, 26], 128),                 # heads that fill no quad; 31 tokens, an empty row
+    (16, 2, [33], 136),                      # 33 tokens: 8 waves a token; strided heads
+    (6, 6, [100, 156], 130),                 # head rows 4-byte but not 8-byte aligned: the narrow loads
+    (32, 8, [257], 128),                     # 257 tokens: 4 waves a token, a last workgroup of its own
+    (5, 1, [300, 1, 900], 128),
+])
+@pytest.mark.parametrize("norm", [True, False])
+def test_fused_edges_match_oracle(gpu, hq, hkv, lens, width, norm):
+    """Head counts and token counts at the edges of the kernel's quads, waves and workgroups, wide and
+    narrow loads, with the norm and permute and without, two padding tokens past the last row."""
+    say("fused edges", hq, hkv, lens, width, norm)
+    ctx = [n + 21 * (i + 1) if n else 0 for i, n in enumerate(lens)]
+    step = build_step(hq=hq, hkv=hkv, ctx_len=ctx, q_len=lens, is_draft=[0] * len(lens), draft_budget=0, seed=17,
+                      device=gpu, bucket_tokens=sum(lens) + 2)
+    g = torch.Generator().manual_seed(23)
+    T = step.total_tokens
+    pad = lambda h: torch.randn(T + 2, h, width, generator=g).to(torch.bfloat16)
+    qf, kf, v = pad(hq), pad(hkv), torch.randn(T + 2, hkv, 128, generator=g).to(torch.bfloat16)
+    q, k = qf[:, :, :128], kf[:, :, :128]
+    w = (torch.rand(2, 128, generator=g) + 0.5).to(torch.bfloat16) if norm else (None, None)
+    offsets = torch.from_numpy(np.append(step.ctx_len - step.q_len, 0).astype(np.int32))
+    before = step.cache.cpu()
+    cache = step.cache.clone()
+    qd, kd = qf.to(gpu), kf.to(gpu)
+    args = [t.to(gpu) if t is not None else None for t in w]
+    qk_norm_rope_update_kv(qd[:, :, :128], kd[:, :, :128], v.to(gpu), *args, 1e-6, step.qo_indptr, offsets.to(gpu),
+                           cache, step.kv_indices, step.kv_indptr, step.last_page_len, PAGE, config=RopeConfig(1e6))
+    torch.cuda.synchronize()
+    ref_q, ref_k = qk_norm_rope(q, k, step.qo_indptr_host.numpy()[:-1], offsets.numpy()[:-1], theta=1e6,
+                                q_weight=w[0], k_weight=w[1], eps=1e-6)
+    pairs_close(qd[:T, :, :128], ref_q[:T])
+    assert torch.equal(qd[:, :, 128:].cpu(), qf[:, :, 128:]) and torch.equal(kd.cpu(), kf)
+    ref = paged_kv_append(bits(ref_k), bits(v), step.qo_indptr_host.numpy()[:-1], bits(before),
+                          step.kv_indices.cpu().numpy(), step.kv_indptr_host.numpy()[:-1],
+                          step.last_page_len.cpu().numpy()[:-1], PAGE)
+    ref = torch.from_numpy(ref.view(np.int16)).view(torch.bfloat16)
+    got = cache.cpu()
+    assert torch.equal(got[:, 1], ref[:, 1])              # V: exact copies, nothing else touched
+    changed = (ref[:, 0] != before[:, 0]).any(dim=-1)
+    assert torch.equal(got[:, 0][~changed], before[:, 0][~changed])
+    pairs_close(got[:, 0][changed], ref[:, 0][changed])
