@@ -39,6 +39,7 @@ EXPORTED = (
     "aspire_host_plan_reset",
     "aspire_host_plan_step",
     "aspire_qk_norm_rope_append",
+    "aspire_qk_norm_rope_append_partials",
     "aspire_rope_frequencies",
     "aspire_build_head_page_lists",
     "aspire_plan_build_segments",
@@ -53,6 +54,10 @@ EXPORTED = (
     "aspire_verify_topk_speculation",
     "aspire_prefill_block_tokens",
     "aspire_prefill_run",
+    "aspire_linear",
+    "aspire_linear_splits",
+    "aspire_linear_partials",
+    "aspire_add_rms_norm_partials",
     "aspire_bandwidth_probe",
 )
 
@@ -204,6 +209,7 @@ def _declare(lib):
         "aspire_host_plan_step": [ctypes.POINTER(HostPlanConfig), ctypes.POINTER(HostPlanStateC),
                                   ctypes.POINTER(HostPlanInputs), ctypes.POINTER(HostPlanOutputs)],
         "aspire_qk_norm_rope_append": [ctypes.POINTER(RopeArgs), vp],
+        "aspire_qk_norm_rope_append_partials": [ctypes.POINTER(RopeArgs), vp, i32, vp],
         "aspire_rope_frequencies": [i32, f32, f32, i32, f32, f32, f32, vp],
         "aspire_build_head_page_lists": [vp, i32, vp, i64, vp, vp, i64, i64, vp, i32, i32, i32, vp, i64, vp, i32,
                                          vp],
@@ -219,6 +225,10 @@ def _declare(lib):
         "aspire_verify_topk_speculation": [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp],
         "aspire_prefill_block_tokens": [i32, i32],
         "aspire_prefill_run": [ctypes.POINTER(PrefillArgs), vp],
+        "aspire_linear": [vp, i64, vp, i64, vp, i64, i32, i32, i32, i32, vp],
+        "aspire_linear_splits": [i32, i32, i32],
+        "aspire_linear_partials": [vp, i64, vp, i64, vp, i64, i32, i32, i32, vp],
+        "aspire_add_rms_norm_partials": [vp, i64, vp, i32, vp, vp, i64, i32, i32, f32, vp],
         "aspire_bandwidth_probe": [i32, vp, i64, vp, i64, i32, i32, vp],
     }
     for name, argtypes in sigs.items():

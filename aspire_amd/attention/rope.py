@@ -57,7 +57,7 @@ def _i32(t):
 
 def _run(q, k, indptr, offsets, *, config, v=None, q_norm_weight=None, k_norm_weight=None, eps=1e-6,
          permute=True, kv_cache=None, kv_page_indices=None, kv_page_indptr=None, kv_last_page_len=None,
-         page_size=16, write_k=True, what="rope"):
+         page_size=16, write_k=True, partials=None, num_kv_heads=0, what="rope"):
     T = q.shape[0]
     if T == 0:
         return
@@ -65,13 +65,17 @@ def _run(q, k, indptr, offsets, *, config, v=None, q_norm_weight=None, k_norm_we
     for name, t in (("q", q), ("k", k), ("v", v)):
         if t is not None and (t.dtype != torch.bfloat16 or t.dim() != 3 or t.shape[-1] != 128 or t.stride(-1) != 1):
             raise ValueError(f"{what}: {name} must be bf16 [T, H, 128] with contiguous head dims")
-    if k.shape[0] != T or (v is not None and v.shape[0] != T):
-        raise ValueError(f"{what}: q, k and v must have the same number of tokens")
+    if partials is None:
+        num_kv_heads = k.shape[1]
+        if k.shape[0] != T or (v is not None and v.shape[0] != T):
+            raise ValueError(f"{what}: q, k and v must have the same number of tokens")
     ind, off = _i32(indptr), _i32(offsets)
     rows = min(ind.shape[0] - 1, off.shape[0])
     a = _lib.RopeArgs()
     a.q, a.q_stride_t, a.q_stride_h, a.num_qo_heads = q.data_ptr(), q.stride(0), q.stride(1), q.shape[1]
-    a.k, a.k_stride_t, a.k_stride_h, a.num_kv_heads = k.data_ptr(), k.stride(0), k.stride(1), k.shape[1]
+    a.num_kv_heads = num_kv_heads
+    if k is not None:
+        a.k, a.k_stride_t, a.k_stride_h = k.data_ptr(), k.stride(0), k.stride(1)
     if v is not None:
         a.v, a.v_stride_t, a.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
     a.total_tokens, a.head_dim = T, 128
@@ -99,7 +103,12 @@ def _run(q, k, indptr, offsets, *, config, v=None, q_norm_weight=None, k_norm_we
         a.kv_page_indices, a.kv_page_indptr, a.kv_last_page_len = pi.data_ptr(), pp.data_ptr(), lp.data_ptr()
         a.num_seq = lp.shape[0]
     a.write_k = int(write_k)
-    _lib.check(_lib.lib().aspire_qk_norm_rope_append(ctypes.byref(a), _lib.stream_of(q)), what)
+    if partials is None:
+        rc = _lib.lib().aspire_qk_norm_rope_append(ctypes.byref(a), _lib.stream_of(q))
+    else:
+        rc = _lib.lib().aspire_qk_norm_rope_append_partials(ctypes.byref(a), _lib.ptr(partials), partials.shape[0],
+                                                            _lib.stream_of(q))
+    _lib.check(rc, what)
 
 
 def apply_rope_inplace(q, k, indptr, offsets, config: RopeConfig | None = None) -> None:
@@ -115,6 +124,26 @@ def qk_norm_rope_update_kv(q, k, v, q_norm_weight, k_norm_weight, eps, kv_append
          k_norm_weight=k_norm_weight, eps=eps, permute=permute, kv_cache=kv_cache, kv_page_indices=kv_page_indices,
          kv_page_indptr=kv_page_indptr, kv_last_page_len=kv_last_page_len, page_size=page_size,
          write_k=False, what="mylib::qk_norm_rope_update_kv")
+
+
+def qk_norm_rope_update_kv_partials(partials, q, num_kv_heads, q_norm_weight, k_norm_weight, eps, kv_append_indptr,
+                                    offsets, kv_cache, kv_page_indices, kv_page_indptr, kv_last_page_len, page_size,
+                                    config: RopeConfig | None = None, permute: bool = True) -> None:
+    """``qk_norm_rope_update_kv`` of a projection that is still split: ``partials`` ``[S, T, (Hq + 2 Hkv) * 128]``
+    fp32 (``linear_partials`` over weight rows in q, k, v order), whose sum over ``S`` is rounded once to
+    bf16; the prepared q goes to ``q`` ``[T, Hq, 128]``."""
+    what = "qk_norm_rope_update_kv_partials"
+    if partials.dtype != torch.float32 or partials.dim() != 3 or not partials.is_contiguous() \
+            or tuple(partials.shape[1:]) != (q.shape[0], (q.shape[1] + 2 * num_kv_heads) * 128):
+        raise ValueError(f"{what}: partials must be contiguous fp32 [S, T, (Hq + 2 * Hkv) * 128]")
+    _lib.require_cuda(partials, kv_cache, what=what)
+    # the kernel reads the norm weights 8 bytes at a time
+    q_norm_weight, k_norm_weight = (w.clone() if w is not None and w.data_ptr() % 8 else w
+                                    for w in (q_norm_weight, k_norm_weight))
+    _run(q, None, kv_append_indptr, offsets, config=config or _CONFIG, q_norm_weight=q_norm_weight,
+         k_norm_weight=k_norm_weight, eps=eps, permute=permute, kv_cache=kv_cache, kv_page_indices=kv_page_indices,
+         kv_page_indptr=kv_page_indptr, kv_last_page_len=kv_last_page_len, page_size=page_size, write_k=False,
+         partials=partials, num_kv_heads=num_kv_heads, what=what)
 
 
 _DEFINED = False
@@ -157,4 +186,5 @@ def define_rope_op(rope_base: float, scaling_factor: float = 1.0, low_freq_facto
     _DEFINED = True
 
 
-__all__ = ["RopeConfig", "rope_frequencies", "apply_rope_inplace", "qk_norm_rope_update_kv", "define_rope_op"]
+__all__ = ["RopeConfig", "rope_frequencies", "apply_rope_inplace", "qk_norm_rope_update_kv",
+           "qk_norm_rope_update_kv_partials", "define_rope_op"]

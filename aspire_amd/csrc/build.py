@@ -23,7 +23,7 @@ LIB = PKG / "libaspire_hip.so"
 BUILD = HERE / "_build"
 SOURCES = ["capi.cpp", "plan.cpp", "host_plan.cpp", "append.hip", "page_list.hip", "attention.hip", "select.hip",
            "rope_append.hip", "decode_ops.hip", "sampling.hip", "prefill.hip",
-           "bandwidth.hip"]
+           "linear.hip", "bandwidth.hip"]
 ARCH = "gfx950"
 
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function"]

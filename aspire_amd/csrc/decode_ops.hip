@@ -24,11 +24,28 @@ __device__ __forceinline__ float bf_round(float f) { return __uint_as_float(bf16
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxChunks = 4;  // dim <= 256 threads * 4 chunks * 8 = 8192
 
-// out[r] = rmsnorm(x[r] (+ delta[r])) * w; with delta, x[r] is updated to the sum.
+// Values 8 i .. 8 i + 7 of row r, summed over the fp32 slabs [splits][rows][dim] of a split linear
+// layer and rounded once to bf16, as that layer's own output would be.
+__device__ __forceinline__ void sum_slabs(const float* partials, int splits, int64_t slab, int64_t at, float* s) {
+  float4 a = *reinterpret_cast<const float4*>(partials + at), b = *reinterpret_cast<const float4*>(partials + at + 4);
+  for (int k = 1; k < splits; ++k) {
+    const float* p = partials + k * slab + at;
+    const float4 c = *reinterpret_cast<const float4*>(p), d = *reinterpret_cast<const float4*>(p + 4);
+    a.x += c.x, a.y += c.y, a.z += c.z, a.w += c.w;
+    b.x += d.x, b.y += d.y, b.z += d.z, b.w += d.w;
+  }
+  s[0] = bf_round(a.x), s[1] = bf_round(a.y), s[2] = bf_round(a.z), s[3] = bf_round(a.w);
+  s[4] = bf_round(b.x), s[5] = bf_round(b.y), s[6] = bf_round(b.z), s[7] = bf_round(b.w);
+}
+
+// out[r] = rmsnorm(x[r] (+ delta[r])) * w; with delta (bf16 rows, or the slabs of a split linear
+// layer), x[r] is updated to the sum. Latency-bound at decode sizes: one launch also takes the slabs'
+// sum, which the layer would otherwise need a launch of its own for.
 __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(uint16_t* x, const uint16_t* delta,
                                                                      const uint16_t* w, uint16_t* out, int dim,
                                                                      int64_t x_stride, int64_t d_stride,
-                                                                     int64_t o_stride, float eps) {
+                                                                     int64_t o_stride, float eps, const float* slabs,
+                                                                     int splits) {
   __shared__ float partial[kNormThreads / 64];
   const int r = blockIdx.x;
   uint4* xr = reinterpret_cast<uint4*>(x + int64_t(r) * x_stride);
@@ -64,9 +81,16 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(uint16_t* x,
           s[2 * e] = bf_round(s[2 * e] + bf_lo(bw[e]));
           s[2 * e + 1] = bf_round(s[2 * e + 1] + bf_hi(bw[e]));
         }
+      }
+      if (slabs) {
+        float d[8];
+        sum_slabs(slabs, splits, int64_t(gridDim.x) * dim, int64_t(r) * dim + 8 * i, d);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] = bf_round(s[e] + d[e]);
+      }
+      if (dr || slabs)
         xr[i] = make_uint4(pack_bf16x2_exact(s[0], s[1]), pack_bf16x2_exact(s[2], s[3]),
                            pack_bf16x2_exact(s[4], s[5]), pack_bf16x2_exact(s[6], s[7]));
-      }
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         v[c][e] = s[e];
@@ -199,7 +223,28 @@ extern "C" int aspire_add_rms_norm(void* x, int64_t x_stride, const void* delta,
   hipLaunchKernelGGL(add_rms_norm_kernel, dim3(rows), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
                      static_cast<uint16_t*>(x), static_cast<const uint16_t*>(delta),
                      static_cast<const uint16_t*>(weight), static_cast<uint16_t*>(out), dim, x_stride,
-                     delta_stride, out_stride, eps);
+                     delta_stride, out_stride, eps, static_cast<const float*>(nullptr), 0);
+  ASPIRE_CHECK_LAUNCH();
+  return ASPIRE_OK;
+}
+
+extern "C" int aspire_add_rms_norm_partials(void* x, int64_t x_stride, const float* partials, int32_t splits,
+                                            const void* weight, void* out, int64_t out_stride, int32_t rows,
+                                            int32_t dim, float eps, void* stream) {
+  using namespace aspire;
+  ASPIRE_CHECK_ARG(rows >= 0, "negative rows");
+  if (rows == 0) return ASPIRE_OK;
+  ASPIRE_CHECK_ARG(x && weight && out && partials && splits >= 1, "null pointer or no partials");
+  ASPIRE_CHECK_ARG(dim > 0 && dim % 8 == 0 && dim <= kNormThreads * kNormMaxChunks * 8,
+                   "dim must be a multiple of 8 and at most 8192");
+  ASPIRE_CHECK_ARG(aligned16(x) && aligned16(weight) && aligned16(out) && aligned16(partials),
+                   "rows must be 16-byte aligned");
+  ASPIRE_CHECK_ARG(x_stride % 8 == 0 && out_stride % 8 == 0 && x_stride >= dim && out_stride >= dim,
+                   "row strides must be multiples of 8 elements and at least dim");
+  hipLaunchKernelGGL(add_rms_norm_kernel, dim3(rows), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
+                     static_cast<uint16_t*>(x), static_cast<const uint16_t*>(nullptr),
+                     static_cast<const uint16_t*>(weight), static_cast<uint16_t*>(out), dim, x_stride, int64_t(0),
+                     out_stride, eps, partials, splits);
   ASPIRE_CHECK_LAUNCH();
   return ASPIRE_OK;
 }

@@ -50,6 +50,8 @@ struct RopeParams {
   const int32_t* last_page_len;
   int32_t num_seq;
   int32_t write_k;
+  const float* partials;  // fp32 slabs [splits][T][(hq + 2 hkv) * 128] of the fused projection, or null
+  int32_t splits;
 };
 
 // Head slots of one wave pass: 4 groups of 16 lanes, one head each.
@@ -80,6 +82,18 @@ __device__ __forceinline__ uint4 load_lane_dims(const uint16_t* row, int j, bool
   auto word = [&](int d) { return uint32_t(row[d]) | (uint32_t(row[d + 1]) << 16); };
   return make_uint4(word(d0), word(d0 + 2), word(d1), word(d1 + 2));
 }
+// The same words from a row of fp32 slabs: summed, and rounded once as the projection's output would be.
+__device__ __forceinline__ uint4 sum_lane_dims(const float* row, int splits, int64_t slab, int j, bool permute) {
+  const int d0 = permute ? 4 * j : 8 * j, d1 = permute ? kPairs + 4 * j : 8 * j + 4;
+  float4 a = *reinterpret_cast<const float4*>(row + d0), b = *reinterpret_cast<const float4*>(row + d1);
+  for (int k = 1; k < splits; ++k) {
+    row += slab;
+    const float4 c = *reinterpret_cast<const float4*>(row + d0), d = *reinterpret_cast<const float4*>(row + d1);
+    a.x += c.x, a.y += c.y, a.z += c.z, a.w += c.w;
+    b.x += d.x, b.y += d.y, b.z += d.z, b.w += d.w;
+  }
+  return make_uint4(pack_bf16x2_rne(a.x, a.y), pack_bf16x2_rne(a.z, a.w), pack_bf16x2_rne(b.x, b.y), pack_bf16x2_rne(b.z, b.w));
+}
 __device__ __forceinline__ void split_pairs(const uint4& w, bool permute, float* a, float* b) {
   if (permute) {
     a[0] = lo_bf(w.x), a[1] = hi_bf(w.x), a[2] = lo_bf(w.y), a[3] = hi_bf(w.y);
@@ -104,7 +118,8 @@ __device__ __forceinline__ void round_pair(float& x, float& y) {
 // loads, two searches and a sincosf for every head took 168 us for 8,192 tokens of 32 q / 8 kv
 // heads (1.2 TB/s, bound by the sincosf and address arithmetic) where this takes 48 us (4.2 TB/s);
 // 208 tokens 6.3 -> 4.8 us.
-template <bool kWide>
+// kSum: the inputs are the slabs of a split projection; q is written to p.q, nothing is read from it.
+template <bool kWide, bool kSum>
 __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(RopeParams p, int total_tokens, int wpt_log2) {
   __shared__ float2 rot[kRopeWaves][kPairs];
   const int lane = threadIdx.x & 63;
@@ -122,7 +137,11 @@ __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(Ro
   // a head's words: q / k dims for the rotation, 16 bytes of v for the copy
   auto load = [&](int h) -> uint4 {
     uint4 w = make_uint4(0, 0, 0, 0);
-    if (h < p.hq) {
+    if (kSum) {
+      const int64_t width = int64_t(p.hq + 2 * p.hkv) * kHeadDim;
+      if (h < n_all)
+        w = sum_lane_dims(p.partials + tok * width + h * kHeadDim, p.splits, total_tokens * width, j, permute && h < n_qk);
+    } else if (h < p.hq) {
       w = load_lane_dims<kWide>(p.q + int64_t(tok) * p.q_st + int64_t(h) * p.q_sh, j, permute);
     } else if (h < n_qk) {
       w = load_lane_dims<kWide>(p.k + int64_t(tok) * p.k_st + int64_t(h - p.hq) * p.k_sh, j, permute);
@@ -256,13 +275,15 @@ extern "C" int aspire_rope_frequencies(int32_t head_dim, float rope_theta, float
   return ASPIRE_OK;
 }
 
-extern "C" int aspire_qk_norm_rope_append(const aspire_rope_args* a, void* stream) {
+namespace {
+
+int prepare_qkv(const aspire_rope_args* a, const float* partials, int32_t splits, void* stream) {
   using namespace aspire;
   ASPIRE_CHECK_ARG(a != nullptr, "null arguments");
   ASPIRE_CHECK_ARG(a->head_dim == kHeadDim, "head_dim must be 128");
   ASPIRE_CHECK_ARG(a->total_tokens >= 0 && a->num_qo_heads >= 0 && a->num_kv_heads >= 0, "bad sizes");
   if (a->total_tokens == 0 || a->num_qo_heads + a->num_kv_heads == 0) return ASPIRE_OK;
-  ASPIRE_CHECK_ARG((a->num_qo_heads == 0 || a->q) && (a->num_kv_heads == 0 || a->k), "null q / k");
+  ASPIRE_CHECK_ARG((a->num_qo_heads == 0 || a->q) && (a->num_kv_heads == 0 || a->k || partials), "null q / k");
   ASPIRE_CHECK_ARG(a->num_rows >= 0 && (a->num_rows == 0 || (a->indptr && a->offsets)), "null indptr / offsets");
   ASPIRE_CHECK_ARG((a->q_norm_weight == nullptr) == (a->k_norm_weight == nullptr),
                    "q and k norm weights go together");
@@ -285,6 +306,8 @@ extern "C" int aspire_qk_norm_rope_append(const aspire_rope_args* a, void* strea
   p.k_w = static_cast<const uint16_t*>(a->k_norm_weight);
   p.eps = a->norm_eps;
   p.permute = a->permute && a->q_norm_weight != nullptr;
+  p.partials = partials;
+  p.splits = splits;
   const int rc = aspire_rope_frequencies(kHeadDim, a->rope_theta, a->rope_scale, a->llama31, a->low_freq_factor,
                                          a->high_freq_factor, a->old_context_len, p.freq);
   if (rc != ASPIRE_OK) return rc;
@@ -309,7 +332,8 @@ extern "C" int aspire_qk_norm_rope_append(const aspire_rope_args* a, void* strea
     ASPIRE_CHECK_ARG(aligned(a->kv_cache, 16) && a->cache_stride_p % 8 == 0 && a->cache_stride_kv % 8 == 0 &&
                          a->cache_stride_t % 8 == 0 && a->cache_stride_h % 8 == 0,
                      "cache must be 16-byte aligned with strides in multiples of 8 elements");
-    ASPIRE_CHECK_ARG(a->v == nullptr || (aligned(a->v, 16) && a->v_stride_t % 8 == 0 && a->v_stride_h % 8 == 0),
+    if (partials != nullptr) p.v = reinterpret_cast<const uint16_t*>(partials);  // the v heads follow in the slabs
+    ASPIRE_CHECK_ARG(partials != nullptr || a->v == nullptr || (aligned(a->v, 16) && a->v_stride_t % 8 == 0 && a->v_stride_h % 8 == 0),
                      "v rows must be 16-byte aligned");
   }
   const bool wide = aligned(a->q, 16) && aligned(a->k, 16) && aligned(p.q_w, 8) && aligned(p.k_w, 8) &&
@@ -320,11 +344,27 @@ extern "C" int aspire_qk_norm_rope_append(const aspire_rope_args* a, void* strea
   // 3.9 / 4.3 / 4.9, 208: 5.0 / 4.8 / 5.2, 512: 7.9 / 7.0 / 6.4, 8,192: 81 / 62 / 48; with 16 / 8
   // heads 80: 3.9 / 3.6 / 4.2, 304: 5.5 / 4.4 / 4.7, 512: 7.7 / 5.1 / 5.1.
   const int wpt_log2 = a->total_tokens <= 32 ? 4 : a->total_tokens <= 256 ? 3 : 2;
+  ASPIRE_CHECK_ARG(partials == nullptr || (p.cache != nullptr && wide && aligned(partials, 16) && splits >= 1 && !a->write_k),
+                   "partials need a cache, 16-byte aligned slabs and q rows, and write_k 0");
   const int64_t units = int64_t(a->total_tokens) << wpt_log2;
   const dim3 grid(unsigned((units + kRopeWaves - 1) / kRopeWaves));
-  const auto kernel = wide ? qk_norm_rope_append_kernel<true> : qk_norm_rope_append_kernel<false>;
+  const auto kernel = p.partials ? qk_norm_rope_append_kernel<true, true>
+                      : wide     ? qk_norm_rope_append_kernel<true, false>
+                                 : qk_norm_rope_append_kernel<false, false>;
   hipLaunchKernelGGL(kernel, grid, dim3(64 * kRopeWaves), 0, static_cast<hipStream_t>(stream), p, a->total_tokens,
                      wpt_log2);
   ASPIRE_CHECK_LAUNCH();
   return ASPIRE_OK;
+}
+
+}  // namespace
+
+extern "C" int aspire_qk_norm_rope_append(const aspire_rope_args* a, void* stream) {
+  return prepare_qkv(a, nullptr, 0, stream);
+}
+
+extern "C" int aspire_qk_norm_rope_append_partials(const aspire_rope_args* a, const float* partials, int32_t splits,
+                                                   void* stream) {
+  if (partials == nullptr) return aspire::fail(ASPIRE_ERR_INVALID, "aspire_qk_norm_rope_append_partials: null partials");
+  return prepare_qkv(a, partials, splits, stream);
 }

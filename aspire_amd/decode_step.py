@@ -11,11 +11,16 @@ The step follows ``TransformerSparseDraft.unified_forward``
                f = ffn_norm(x); x += w2(silu(w1 f) * w3 f)
     logits = output(norm(x)); ids = argmax(logits)
 
-The GEMMs are torch's (hipBLASLt). The q/k preparation and the append are one
-launch (``qk_norm_rope_update_kv``), the attention is ``HolisticAttentionWrapper``,
-and the residual adds, norms, SwiGLU step and token pick are the row kernels of
-the HIP library (``aspire_add_rms_norm``, ``aspire_silu_mul``,
-``aspire_argmax_rows``), so a whole step can be recorded in one HIP graph.
+Steps of at most ``linear.MAX_ROWS`` tokens run their projections on the HIP
+library's own kernels (``aspire_amd.linear``): w13 with the SwiGLU step in its
+epilogue, and wqkv, wo and w2 split over K, their fp32 partial sums taken by the
+launch that follows anyway (the q/k preparation, the residual add + norm). Larger
+steps use torch's GEMMs (hipBLASLt), as does the vocabulary projection past
+``HEAD_ROWS`` tokens. The q/k preparation and the append are one launch
+(``qk_norm_rope_update_kv``), the attention is ``HolisticAttentionWrapper``, and
+the residual adds, norms and token pick are the row kernels of the HIP library
+(``aspire_add_rms_norm``, ``aspire_argmax_rows``), so a whole step can be
+recorded in one HIP graph.
 
 Refresh layer, ``selector="keymean"`` (BASELINE config 2's selection): at
 ``refresh_layer`` every row attends its full context and the kernel writes the
@@ -47,13 +52,17 @@ import torch
 import torch.nn.functional as F
 
 from aspire_amd import _lib
+from aspire_amd import linear as lin
 from aspire_amd.attention.holistic_wrapper import HolisticAttentionWrapper, build_holistic_dump_jit_args
 from aspire_amd.attention.page_list import build_head_page_lists, build_unified_indices
-from aspire_amd.attention.rope import RopeConfig, qk_norm_rope_update_kv
+from aspire_amd.attention.rope import RopeConfig, qk_norm_rope_update_kv, qk_norm_rope_update_kv_partials
 from aspire_amd.backends.page_selector import KeyMeanPageSelector, PageSelectorFirstLastAvg
 
 PAGE = 16
 DRAFT_MODE, VERIFY_MODE = 0, 1
+# Tokens up to which the vocabulary projection runs on aspire_linear: at 151,936 x 4,096 it takes 196 us
+# at 12 rows, 210 at 48 and 249 at 104 where hipBLASLt takes 244, 262 and 277, but 355 against 324 at 208.
+HEAD_ROWS = 128
 
 
 @dataclass(frozen=True)
@@ -113,6 +122,26 @@ def add_rms_norm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, eps: 
         _lib.ptr(x), x.stride(0), _lib.ptr(delta), delta.stride(0) if delta is not None else 0, _lib.ptr(weight),
         _lib.ptr(out), out.stride(0), x.shape[0], x.shape[1], float(eps), _lib.stream_of(x))
     _lib.check(rc, "add_rms_norm")
+    return out
+
+
+def add_rms_norm_partials(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, eps: float,
+                          partials: torch.Tensor) -> torch.Tensor:
+    """``add_rms_norm`` with ``delta`` the bf16-rounded sum of ``partials`` ``[S, rows, dim]`` fp32."""
+    _lib.require_cuda(x, weight, out, partials, what="add_rms_norm_partials")
+    _bf16_rows(x, "x")
+    _bf16_rows(out, "out")
+    if weight.dtype != torch.bfloat16 or not weight.is_contiguous() or weight.numel() != x.shape[1]:
+        raise ValueError("add_rms_norm_partials: weight must be a contiguous bf16 vector of x's width")
+    if out.shape != x.shape:
+        raise ValueError("add_rms_norm_partials: out must match x")
+    if partials.dtype != torch.float32 or not partials.is_contiguous() or partials.dim() != 3 \
+            or partials.shape[1:] != x.shape or partials.shape[0] < 1:
+        raise ValueError("add_rms_norm_partials: partials must be contiguous fp32 [S, rows, dim]")
+    rc = _lib.lib().aspire_add_rms_norm_partials(_lib.ptr(x), x.stride(0), _lib.ptr(partials), partials.shape[0],
+                                                 _lib.ptr(weight), _lib.ptr(out), out.stride(0), x.shape[0], x.shape[1],
+                                                 float(eps), _lib.stream_of(x))
+    _lib.check(rc, "add_rms_norm_partials")
     return out
 
 
@@ -365,6 +394,12 @@ class MixedDecodeStep:
         self.act = torch.empty(T, shape.intermediate_size, dtype=bf, device=dev)
         self.ids = torch.zeros(T, dtype=torch.int64, device=dev)
         self.logits = None
+        # partial sums of whichever projection waits for its consumer (see _project)
+        sizes = ((shape.q_size + 2 * shape.kv_size, shape.dim), (shape.dim, shape.q_size),
+                 (shape.dim, shape.intermediate_size))
+        self.partials = torch.empty(max(lin.linear_splits(T, n, k) * T * n for n, k in sizes), dtype=torch.float32,
+                                    device=dev)
+        self.q = torch.empty(T, shape.n_head, shape.head_dim, dtype=bf, device=dev)
 
         self.build_lists()
         # plan() once (the wrappers' module set-up, as the reference requires before plan_host)
@@ -438,39 +473,64 @@ class MixedDecodeStep:
         (after RoPE) as ``q{layer}``, the attention output as ``y{layer}`` and the
         final hidden state as ``h``."""
         s, w = self.shape, self.w
-        T = self.T
-        qs, kvs = s.q_size, s.kv_size
         self._full_lists()
         if self.selector_kind == "first_last":
             self.select_first_last()
         torch.index_select(w.tok_embeddings, 0, self.tokens, out=self.x)
-        ffn_out = None
+        pending = None  # the previous block's output, not yet added to x
         for layer, lw in enumerate(w.layers):
-            add_rms_norm(self.x, lw["attention_norm"], self.a, s.norm_eps, delta=ffn_out)
-            qkv = F.linear(self.a, lw["wqkv"])
-            q = qkv[:, :qs].view(T, s.n_head, s.head_dim)
-            k = qkv[:, qs : qs + kvs].view(T, s.n_local_heads, s.head_dim)
-            v = qkv[:, qs + kvs :].view(T, s.n_local_heads, s.head_dim)
-            if capture is not None:
-                capture[f"qkv{layer}"] = qkv.clone()  # q is rewritten in place below
-            qk_norm_rope_update_kv(q, k, v, lw["q_norm"], lw["k_norm"], s.norm_eps, self.qo_indptr, self.offsets,
-                                   self.caches[layer], self.full_indices, self.full_indptr, self.last_page_len, PAGE,
-                                   config=self.rope)
+            self._add_norm(lw["attention_norm"], pending)
+            qkv = self._project(self.a, lw["wqkv"])
+            if capture is not None:  # q is rewritten in place below
+                capture[f"qkv{layer}"] = qkv.clone() if qkv.dim() == 2 else qkv.sum(0).to(torch.bfloat16)
+            q = self._prepare_qkv(layer, lw, qkv)
             if capture is not None:
                 capture[f"q{layer}"] = q.clone()
             self.attention(layer, q)
             if capture is not None:
                 capture[f"y{layer}"] = self.y.clone()
-            attn_out = F.linear(self.y.view(T, qs), lw["wo"])
-            add_rms_norm(self.x, lw["ffn_norm"], self.a, s.norm_eps, delta=attn_out)
-            gate_up = F.linear(self.a, lw["w13"])
-            silu_mul(gate_up, self.act)
-            ffn_out = F.linear(self.act, lw["w2"])
-        add_rms_norm(self.x, w.norm, self.a, s.norm_eps, delta=ffn_out)
+            self._add_norm(lw["ffn_norm"], self._project(self.y.view(self.T, s.q_size), lw["wo"]))
+            if lin.supported(self.a, lw["w13"]):
+                lin.linear(self.a, lw["w13"], self.act, swiglu=True)
+            else:
+                silu_mul(F.linear(self.a, lw["w13"]), self.act)
+            pending = self._project(self.act, lw["w2"])
+        self._add_norm(w.norm, pending)
         if capture is not None:
             capture["h"] = self.a.clone()
-        self.logits = F.linear(self.a, w.output)
+        if self.T <= HEAD_ROWS and lin.supported(self.a, w.output):
+            self.logits = lin.linear(self.a, w.output, torch.empty(self.T, w.output.shape[0], dtype=self.a.dtype,
+                                                                   device=self.device))
+        else:
+            self.logits = F.linear(self.a, w.output)
         return argmax_rows(self.logits, self.ids)
+
+    def _project(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """``x @ w.T``: its split partial sums ``[S, T, N]`` fp32 (in ``partials``, until the next call) where
+        the library's kernels take the shape, else the bf16 ``[T, N]`` of torch's GEMM."""
+        return lin.linear_partials(x, w, self.partials) if lin.supported(x, w) else F.linear(x, w)
+
+    def _add_norm(self, weight: torch.Tensor, delta: torch.Tensor | None) -> None:
+        """``x += delta`` (a ``_project`` result), ``a = RMSNorm(x) * weight``."""
+        if delta is not None and delta.dim() == 3:
+            add_rms_norm_partials(self.x, weight, self.a, self.shape.norm_eps, delta)
+        else:
+            add_rms_norm(self.x, weight, self.a, self.shape.norm_eps, delta=delta)
+
+    def _prepare_qkv(self, layer: int, lw: dict, qkv: torch.Tensor) -> torch.Tensor:
+        """q/k norm, RoPE and the append of a layer's fused projection; the prepared q."""
+        s, T = self.shape, self.T
+        args = (lw["q_norm"], lw["k_norm"], s.norm_eps, self.qo_indptr, self.offsets, self.caches[layer],
+                self.full_indices, self.full_indptr, self.last_page_len, PAGE)
+        if qkv.dim() == 3:
+            qk_norm_rope_update_kv_partials(qkv, self.q, s.n_local_heads, *args, config=self.rope)
+            return self.q
+        qs, kvs = s.q_size, s.kv_size
+        q = qkv[:, :qs].view(T, s.n_head, s.head_dim)
+        k = qkv[:, qs : qs + kvs].view(T, s.n_local_heads, s.head_dim)
+        v = qkv[:, qs + kvs :].view(T, s.n_local_heads, s.head_dim)
+        qk_norm_rope_update_kv(q, k, v, *args, config=self.rope)
+        return q
 
     def attention_only(self) -> None:
         """The step's attention work alone (for the attention share): both list builds,

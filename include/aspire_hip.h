@@ -410,6 +410,12 @@ typedef struct aspire_rope_args {
 
 int aspire_qk_norm_rope_append(const aspire_rope_args* args, void* stream);
 
+/* The same from the fp32 slabs [splits][T][(Hq + 2 Hkv) * 128] of a split fused projection
+ * (aspire_linear_partials with w's rows in q, k, v order): q, k and v are bf16(the slabs' sum). args'
+ * k and v are not read, q is written only (16-byte aligned rows), a cache is needed and write_k is 0. */
+int aspire_qk_norm_rope_append_partials(const aspire_rope_args* args, const float* partials, int32_t splits,
+                                        void* stream);
+
 /* The head_dim / 2 fp32 rotary frequencies the kernel uses (host only):
  * theta^(-2i/head_dim) / rope_scale, or the Llama 3.1 smoothing. */
 int aspire_rope_frequencies(int32_t head_dim, float rope_theta, float rope_scale, int32_t llama31,
@@ -434,6 +440,25 @@ int aspire_add_rms_norm(void* x, int64_t x_stride, const void* delta, int64_t de
  * gate (w1) and up (w3) projections side by side in one row. */
 int aspire_silu_mul(const void* gate_up, int64_t gate_up_stride, void* out, int64_t out_stride,
                     int32_t rows, int32_t inter, void* stream);
+
+/* A linear layer of a few token rows: out[m, n] = bf16(sum_k x[m, k] * w[n, k]), fp32 accumulation
+ * (the nn.Linear calls of the mixed forward, transformer.py:490-502, sparse_draft_transformer.py:149-177,
+ * 276). With swiglu, w holds n gate rows then n up rows and out[m, :n] = silu(gate) * up with
+ * aspire_silu_mul's roundings. rows <= 224, k % 128 == 0, n % 16 == 0, 16-byte aligned rows of x and w. */
+int aspire_linear(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out,
+                  int64_t out_stride, int32_t rows, int32_t n, int32_t k, int32_t swiglu, void* stream);
+
+/* The same layer with k split: partials [splits][rows][n] fp32, whose sum over the slabs is the output,
+ * for a consumer that reads it once (aspire_add_rms_norm_partials, aspire_rope_args.partials).
+ * aspire_linear_splits says how many slabs a shape takes (0: refused; host only). */
+int32_t aspire_linear_splits(int32_t rows, int32_t n, int32_t k);
+int aspire_linear_partials(const void* x, int64_t x_stride, const void* w, int64_t w_stride, float* partials,
+                           int64_t partials_size, int32_t rows, int32_t n, int32_t k, void* stream);
+
+/* aspire_add_rms_norm with delta = bf16(the sum of the slabs partials [splits][rows][dim]). */
+int aspire_add_rms_norm_partials(void* x, int64_t x_stride, const float* partials, int32_t splits,
+                                 const void* weight, void* out, int64_t out_stride, int32_t rows, int32_t dim,
+                                 float eps, void* stream);
 
 /* Greedy token pick (the top_k == 0 branch of TransformerSparseDraft.unified_forward,
  * sparse_draft_transformer.py:276-286): ids[r] = the first index of the
