@@ -84,6 +84,52 @@ def test_topk_candidates_paths(gpu, case):
     assert torch.equal(vals.cpu().view(torch.int16), ref_v.view(torch.int16))
 
 
+@pytest.mark.parametrize("vocab,k", [(8192, 1), (8192, 128), (8199, 50), (8191, 50), (151936, 128), (155651, 100)])
+@pytest.mark.parametrize("case", ["random", "few_positive", "ties_512", "ties_513", "signed_zeros", "infinities"])
+def test_topk_by_group_maxima(gpu, vocab, k, case):
+    """Rows the group maxima settle and rows they leave to the radix select: the smallest and largest
+    register-held row, a tail past the last whole vector, fewer positive logits than k, exactly as many
+    ties at the k-th logit as are ranked by counting and one more, zeros of both signs at the k-th
+    place, infinities."""
+    say("topk by maxima", vocab, k, case)
+    g = torch.Generator().manual_seed(vocab + k)
+    x = torch.randn(3, vocab, generator=g) * 2
+    if case == "few_positive":
+        x = -x.abs() - 0.5
+        x[:, torch.randperm(vocab, generator=g)[: max(k - 1, 1)]] = 1.5
+    elif case.startswith("ties"):
+        x = -x.abs() - 1
+        x[:, torch.randperm(vocab, generator=g)[: int(case[5:])]] = 3.0
+    elif case == "signed_zeros":
+        x = -x.abs() - 1
+        at = torch.randperm(vocab, generator=g)
+        x[:, at[:400]] = 0.0
+        x[:, at[400:800]] = -0.0
+        x[:, at[800 : 800 + k // 2]] = 2.0
+    elif case == "infinities":
+        at = torch.randperm(vocab, generator=g)
+        x[:, at[:5]] = float("inf")
+        x[:, at[5:3000]] = float("-inf")
+    x = x.to(torch.bfloat16)
+    vals, ids = local_topk_candidates(x.to(gpu), k, 11)
+    ref_v, ref_i = osamp.topk_candidates(x, k, 11)
+    assert torch.equal(ids.cpu(), ref_i)
+    assert torch.equal(vals.cpu().view(torch.int16), ref_v.view(torch.int16))
+
+
+def test_topk_by_group_maxima_places_nan_as_the_select_does(gpu):
+    """NaN logits of either sign: the first 128 of 129 candidates (radix select) are the 128 candidates
+    (group maxima)."""
+    say("topk nan")
+    g = torch.Generator(device=gpu).manual_seed(4)
+    x = torch.randn(2, 30000, generator=g, device=gpu).to(torch.bfloat16)
+    x[:, 77::5000] = float("nan")
+    x.view(torch.int16)[:, 99::7000] = -1      # a negative NaN
+    v, i = local_topk_candidates(x, 128)
+    rv, ri = local_topk_candidates(x, 129)
+    assert torch.equal(i, ri[:, :128]) and torch.equal(v.view(torch.int16), rv[:, :128].view(torch.int16))
+
+
 def test_merge_topk_candidates(gpu):
     g = torch.Generator().manual_seed(3)
     vals = (torch.randn(6, 4 * 50, generator=g) * 2).round().to(torch.bfloat16)
