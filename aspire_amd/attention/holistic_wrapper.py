@@ -268,6 +268,7 @@ class HolisticAttentionWrapper:
         event.record(stream)
         self._pinned_slot = (slot + 1) % PINNED_RING
 
+        self._plan_host_lens = (qo, kvl)
         self._plan_info = info
         self._plan_tokens = int(qo[: batch + 1].max()) if batch else 0
         # rows that can write dump entries / page scores: queries and at least one page

@@ -4,7 +4,7 @@ The reference plans and runs FlashInfer's paged prefill wrapper for prompt chunk
 (aspire/models/sparse_draft_runner.py:199-209; the chunk loop of ``encode_slots``,
 aspire/backends/base.py:1559-1674): causal attention of each row's new tokens over its
 cached prefix plus the new tokens, page lists as for decode. ``run`` launches the
-dedicated prefill kernel (``aspire_prefill_run``): each workgroup takes one query block
+dedicated prefill kernel (``aspire_prefill_run_units``): each workgroup takes one query block
 (``aspire_prefill_block_tokens(hq, hkv)`` tokens of one row, all G query heads of one kv
 head) and stages every page of its keys once in LDS, two pages per step, for all of its
 waves (head groups that do not divide a wave's 32 query rows take the decode path below).
@@ -32,6 +32,10 @@ import torch
 
 from aspire_amd import _lib
 from aspire_amd.attention.holistic_wrapper import HolisticAttentionWrapper, _unpack_paged_kv_cache
+
+
+# Most memory for the partial outputs of query blocks cut along their keys.
+PARTIAL_BYTES = 256 << 20
 
 
 class BatchPrefillWithPagedKVCacheWrapper(HolisticAttentionWrapper):
@@ -77,22 +81,46 @@ class BatchPrefillWithPagedKVCacheWrapper(HolisticAttentionWrapper):
             # a head group that does not divide a wave's 32 query rows (e.g. 6 or 12 query heads
             # per kv head): the mixed kernel's query tiles serve the plan made above
             return
-        # rows: the entries of kv_last_page_len (FlashInfer's batch), with their query blocks
+        # rows: the entries of kv_last_page_len (FlashInfer's batch), with their query blocks; the
+        # plan above has read the lengths back
         n = paged_kv_last_page_len.shape[0]
-        qo_host = qo_indptr[: n + 1].to("cpu", torch.int64)
-        q_len = (qo_host[1:] - qo_host[:-1]).clamp(min=0)
+        qo_host, kv_len = (t.to(torch.int64) for t in self._plan_host_lens)
+        q_len = (qo_host[1 : n + 1] - qo_host[:n]).clamp(min=0)
         blocks = torch.zeros(n + 1, dtype=torch.int64)
         blocks[1:] = torch.cumsum((q_len + bt - 1) // bt, 0)
         dev = paged_kv_indices.device
+        total = int(blocks[-1])
+        units, merges, slots = self._plan_units(q_len, kv_len[:n], bt, num_qo_heads, num_kv_heads, causal)
+        tables = torch.cat([units.view(-1), merges.view(-1), blocks.to(torch.int32)]).to(dev)  # one upload
+        at = units.numel() + merges.numel()
         self._pf = {
+            "units": tables[: units.numel()].view(-1, 4), "merges": tables[units.numel() : at].view(-1, 4), "slots": slots,
             "qo": qo_indptr[: n + 1].to(dev, torch.int32).contiguous(),
             "kvp": paged_kv_indptr[: n + 1].to(dev, torch.int32).contiguous(),
             "lpl": paged_kv_last_page_len[:n].to(dev, torch.int32).contiguous(),
             "idx": paged_kv_indices.to(torch.int32).contiguous(),
-            "blocks": blocks.to(dev, torch.int32),
-            "rows": n, "total_blocks": int(blocks[-1]), "block_tokens": bt,
-            "tokens": int(qo_host[-1]) if n else 0,
+            "blocks": tables[at:],
+            "rows": n, "total_blocks": total, "block_tokens": bt,
+            "tokens": int(qo_host[n]) if n else 0,
         }
+
+    @staticmethod
+    def _plan_units(q_len, kv_len, block_tokens, num_qo_heads, num_kv_heads, causal):
+        """``(units [U, 4], merges [M, 4], partial slots)`` for the prefill kernel: the query blocks dealt out
+        over the CUs, the long ones cut along their keys where whole blocks would leave the chip idle or uneven."""
+        n = q_len.shape[0]
+        ql, kl = q_len.to(torch.int32).contiguous(), kv_len.to(torch.int32).contiguous()
+        block_rows = block_tokens * num_qo_heads // num_kv_heads
+        most = PARTIAL_BYTES // (num_kv_heads * block_rows * 129 * 4)
+        counts = [ctypes.c_int32() for _ in range(3)]
+        # room for the largest tables: a unit and a merge a block, and every slot a unit
+        blocks = int(((q_len + block_tokens - 1) // block_tokens).sum())
+        table = torch.empty((2 * blocks + most, 4), dtype=torch.int32)
+        rc = _lib.lib().aspire_prefill_plan(_lib.ptr(ql), _lib.ptr(kl), n, num_qo_heads, num_kv_heads, 1 if causal else 0,
+                                            most, _lib.ptr(table), table.numel(), *(ctypes.byref(c) for c in counts))
+        _lib.check(rc, "plan")
+        n_units, n_merges, slots = (c.value for c in counts)
+        return table[:n_units], table[n_units : n_units + n_merges], slots
 
     def run(self, q: torch.Tensor, paged_kv_cache, *args, out: Optional[torch.Tensor] = None,
             lse: Optional[torch.Tensor] = None, return_lse: bool = False, **kwargs):
@@ -140,7 +168,12 @@ class BatchPrefillWithPagedKVCacheWrapper(HolisticAttentionWrapper):
         a.num_qo_heads, a.num_kv_heads, a.head_dim, a.page_size = self._num_qo_heads, self._num_kv_heads, 128, 16
         a.sm_scale = float(self._sm_scale if self._sm_scale is not None else 1.0 / math.sqrt(128))
         a.causal = 1 if self._causal else 0
-        rc = _lib.lib().aspire_prefill_run(ctypes.byref(a), _lib.stream_of(q))
+        # a buffer of this call's own (from torch's pool): runs on several streams do not share it
+        size = pf["slots"] * self._num_kv_heads * (pf["block_tokens"] * self._num_qo_heads // self._num_kv_heads) * 129
+        partials = torch.empty(size, dtype=torch.float32, device=q.device) if size else None
+        rc = _lib.lib().aspire_prefill_run_units(
+            ctypes.byref(a), _lib.ptr(pf["units"]), pf["units"].shape[0], _lib.ptr(pf["merges"]),
+            pf["merges"].shape[0], pf["slots"], _lib.ptr(partials), size, _lib.stream_of(q))
         _lib.check(rc, "BatchPrefillWithPagedKVCacheWrapper.run")
         return (out, lse) if return_lse else out
 

@@ -20,10 +20,20 @@
 //   * O^T += V^T . P^T with 8 v_mfma_f32_16x16x32_bf16 per tile: each lane's 8 keys are
 //     keys 4grp..4grp+3 of both pages (the order S^T left them in), V^T comes from LDS with
 //     transpose reads (ds_read_b64_tr_b16) and is shared by the wave's tiles.
-// The grid is 1-D with the kv head fastest: the last query blocks of every head (the most
-// keys under a causal mask) start first, and with num_kv_heads a multiple of 8 the
-// round-robin spread of workgroups over the 8 XCDs keeps each head's pages in one L2.
+// The grid is 1-D with the kv head fastest: with num_kv_heads a multiple of 8 the round-robin
+// spread of workgroups over the 8 XCDs keeps each head's pages in one L2. aspire_prefill_plan
+// lists the blocks so that the CUs get even shares, and cuts blocks along their keys where whole
+// ones are too few or too long (pieces write normalised fp32 rows and their LSE, merged by
+// prefill_merge_kernel); without a list the last query blocks start first (the most keys under
+// a causal mask). us, one call of 32 / 8 heads: 5 rows of 17 to 700 tokens over 300 to 8,192
+// cached 194 -> 149; 64 tokens over 16,000 332 -> 39, 17 over 30,000 615 -> 42; 4 x 2,048 over 6,144
+// 837 -> 780; 8,192 tokens 463 -> 462.
 // Waves whose tokens end before a step skip its compute but keep staging.
+#include <algorithm>
+#include <functional>
+#include <queue>
+#include <vector>
+
 #include "common.h"
 
 namespace aspire {
@@ -97,6 +107,10 @@ struct PrefillParams {
   int32_t hq, group;
   float scale_log2;
   int32_t causal;
+  // with units: workgroup i * num_kv_heads + g takes steps [begin, end) of unit i's query block
+  const int4* units;  // (query block, begin, end, partial slot or -1: the whole block)
+  float* part_o;      // [slots][num_kv_heads][kPfBlockRows][128] fp32, normalised by the piece's own sum
+  float* part_lse;    // [slots][num_kv_heads][kPfBlockRows], base 2
 };
 
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfWavesPerEu))) void prefill_kernel(
@@ -121,7 +135,10 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
   // multiple of 8, and the last query blocks of every head start first
   const int hkv = p.hq / G;
   const int g = wave_uniform(int(blockIdx.x) % hkv);
-  const int blk = wave_uniform(p.total_blocks - 1 - int(blockIdx.x) / hkv);
+  const int unit = wave_uniform(int(blockIdx.x) / hkv);
+  int4 piece = make_int4(p.total_blocks - 1 - unit, 0, 0x7fffffff, -1);
+  if (p.units != nullptr) piece = p.units[unit];
+  const int blk = wave_uniform(piece.x);
   int lo = 0, hi = p.num_rows - 1, b = 0;
   while (lo <= hi) {
     const int mid = (lo + hi) >> 1;
@@ -149,7 +166,9 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
   const int shift = kv_len - q_len;
   const int blk_last = p.causal ? min(shift + tok0 + ntok - 1, kv_len - 1) : kv_len - 1;
   const int blk_pages = blk_last >= 0 ? blk_last / kPage + 1 : 0;
-  const int steps = wave_uniform((blk_pages + 1) / 2);
+  // this workgroup's steps (a piece's end may lie past the block's last step: the last piece takes them all)
+  const int begin = wave_uniform(piece.y);
+  const int steps = wave_uniform(min((blk_pages + 1) / 2, piece.z));
   const int vlim = wave_uniform(min(kv_len, blk_pages * kPage));
   const int w_last = wave_uniform(rows > 0 ? (p.causal ? min(shift + wt0 + wn - 1, kv_len - 1) : kv_len - 1) : -1);
   const int w_min_limit = wave_uniform(p.causal ? min(shift + wt0, kv_len - 1) : kv_len - 1);
@@ -282,7 +301,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
   // exponentials stay below 2^kPfSlack. They are computed with the current offsets first: a
   // step on which no lane's sum of its 8 exponentials of a row exceeds 2^kPfSlack (so none of
   // them does) keeps them, and only otherwise (and on the first step, which sets every row's
-  // max: key 0 is visible to every row) are the row maxima taken across lanes, the offsets
+  // max: a row that does not see its first key sees none of the piece) are the row maxima taken across lanes, the offsets
   // moved, the accumulators rescaled and the exponentials recomputed (a wave-uniform branch).
   auto softmax = [&](int s) {
     const int key0 = s * kPfStepKeys;
@@ -315,7 +334,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
       }
     };
     exponentials();
-    bool over = s == 0;
+    bool over = s == begin;
 #pragma unroll
     for (int tt = 0; tt < kPfTiles; ++tt) over |= ps[tt] > kPfSumLimit;
     if (__builtin_amdgcn_ballot_w64(over) != 0) {
@@ -371,17 +390,17 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
     pv_update(kb);
   };
 
-  // Pipeline over kPfStages LDS stage buffers (step k in buffer k % kPfStages, separate LDS
+  // Pipeline over kPfStages LDS stage buffers (step begin + k in buffer k % kPfStages, separate LDS
   // objects so the compiler can tell a load into one from a read of another): at the start of
   // step s the loads of step s + kPfStages - 1 go into the buffer step s - 1 used (free since
   // that step's barrier); the barrier at the end of step s waits for step s + 1's loads. Page
   // ids are scalar loads one step ahead of their use. Every step issues the same loads (steps
   // past the block read nothing: every chunk is out of range), so the wait count is the same
   // on every iteration.
-  if (steps > 0) {
+  if (steps > begin) {
 #pragma unroll
-    for (int k = 0; k < kPfStages - 1; ++k) issue(stages[k], k, page_id(k));
-    int next_id = page_id(kPfStages - 1);
+    for (int k = 0; k < kPfStages - 1; ++k) issue(stages[k], begin + k, page_id(begin + k));
+    int next_id = page_id(begin + kPfStages - 1);
     __builtin_amdgcn_s_waitcnt(kPfWait);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -393,7 +412,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
       if (s < steps && s * kPfStepKeys <= w_last) compute(cur, s);
       step_barrier();
     };
-    for (int s = 0; s < steps; s += kPfStages) {
+    for (int s = begin; s < steps; s += kPfStages) {
 #pragma unroll
       for (int u = 0; u < kPfStages; ++u) body(s + u, stages[u], stages[(u + kPfStages - 1) % kPfStages]);
     }
@@ -412,6 +431,18 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
     const int ti = row / G;
     const int head = g * G + (row - ti * G);
     const int token = q0 + wt0 + ti;
+    if (piece.w >= 0) {
+      const int64_t slot = (int64_t(piece.w) * hkv + g) * kPfBlockRows + wave * kPfRows + row;
+      float* dst = p.part_o + slot * kHeadDim;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const f32x4 a = acc[tt][c];
+        *reinterpret_cast<float4*>(dst + 32 * (c >> 1) + 8 * grp + 4 * (c & 1)) =
+            make_float4(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
+      }
+      if (grp == 0) p.part_lse[slot] = lse_v;
+      continue;
+    }
     uint16_t* dst = p.out + int64_t(token) * p.o_st + int64_t(head) * p.o_sh;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -428,6 +459,70 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
   }
 }
 
+// Blocks cut into pieces: out = sum_i 2^(lse_i - m) o_i / sum_i 2^(lse_i - m) over the pieces, rounded
+// once. 16 lanes own a row (8 dims each), 16 rows a workgroup; a round's loads are issued together.
+// HBM- and latency-bound: 512 bytes per row and piece, read once.
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p, const int4* merges) {
+  constexpr int kRound = 4;
+  constexpr int kGroups = kPfBlockRows / 16;
+  const int hkv = p.hq / p.group;
+  const int at = blockIdx.x / kGroups;
+  const int4 m = merges[at / hkv];  // (query block, first slot, pieces)
+  const int g = at % hkv;
+  int b = 0;
+  for (int lo = 0, hi = p.num_rows - 1; lo <= hi;) {
+    const int mid = (lo + hi) >> 1;
+    if (p.block_indptr[mid] <= m.x) {
+      b = mid;
+      lo = mid + 1;
+    } else {
+      hi = mid - 1;
+    }
+  }
+  const int tok0 = (m.x - p.block_indptr[b]) * p.block_tokens;
+  const int q0 = p.qo_indptr[b], q_len = p.qo_indptr[b + 1] - q0;
+  const int row = (blockIdx.x % kGroups) * 16 + (threadIdx.x >> 4), d = (threadIdx.x & 15) * 8;
+  const int ti = row / p.group;
+  if (tok0 + ti >= q_len) return;
+  const int64_t step = int64_t(hkv) * kPfBlockRows;
+  const int64_t first = (int64_t(m.y) * hkv + g) * kPfBlockRows + row;
+  float mx = kNegInfP, sum = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < m.z; k += kRound) {
+    float l[kRound];
+    float4 x[kRound], y[kRound];
+#pragma unroll
+    for (int i = 0; i < kRound; ++i) {
+      const int64_t slot = first + min(k + i, m.z - 1) * step;
+      l[i] = k + i < m.z ? p.part_lse[slot] : kNegInfP;
+      const float4* src = reinterpret_cast<const float4*>(p.part_o + slot * kHeadDim + d);
+      x[i] = src[0];
+      y[i] = src[1];
+    }
+    float top = mx;
+#pragma unroll
+    for (int i = 0; i < kRound; ++i) top = fmaxf(top, l[i]);
+    if (top == kNegInfP) continue;
+    const float keep = __builtin_amdgcn_exp2f(mx - top);
+    sum *= keep;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= keep;
+#pragma unroll
+    for (int i = 0; i < kRound; ++i) {
+      const float w = __builtin_amdgcn_exp2f(l[i] - top);
+      sum += w;
+      o[0] += w * x[i].x, o[1] += w * x[i].y, o[2] += w * x[i].z, o[3] += w * x[i].w;
+      o[4] += w * y[i].x, o[5] += w * y[i].y, o[6] += w * y[i].z, o[7] += w * y[i].w;
+    }
+    mx = top;
+  }
+  const float inv = sum > 0.f ? 1.f / sum : 0.f;
+  const int token = q0 + tok0 + ti, head = g * p.group + (row - ti * p.group);
+  *reinterpret_cast<uint4*>(p.out + int64_t(token) * p.o_st + int64_t(head) * p.o_sh + d) =
+      make_uint4(pack_bf16x2_rne(o[0] * inv, o[1] * inv), pack_bf16x2_rne(o[2] * inv, o[3] * inv),
+                 pack_bf16x2_rne(o[4] * inv, o[5] * inv), pack_bf16x2_rne(o[6] * inv, o[7] * inv));
+  if (d == 0 && p.lse != nullptr) p.lse[int64_t(token) * p.hq + head] = sum > 0.f ? mx + __builtin_log2f(sum) : kNegInfP;
+}
+
 inline bool pf_al16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 }  // namespace
@@ -441,8 +536,80 @@ extern "C" int aspire_prefill_block_tokens(int32_t num_qo_heads, int32_t num_kv_
   return kPfBlockRows / G;
 }
 
-extern "C" int aspire_prefill_run(const aspire_prefill_args* a, void* stream) {
-  using namespace aspire;
+namespace aspire {
+namespace {
+
+constexpr int kPfPerCu = 3;  // workgroups a CU holds
+constexpr int kPfStart = 6;  // a workgroup's start and end, in steps
+
+// Pieces a block of `steps` is cut into at pieces of about `piece` steps (a quarter more stays whole).
+int piece_count(int32_t steps, int64_t piece) {
+  return steps > piece + piece / 4 ? static_cast<int>((steps + piece - 1) / piece) : 1;
+}
+
+// A launch's first workgroups go round a head's CUs one each, then a second and a third each, and only
+// later ones wait for a place. So the units (longest first) are dealt out three a CU, each to the CU
+// with the least work that has a place left, and listed by rounds; the rest follow in their order.
+// Returns the estimated us of the slowest CU: 0.66 us a step for a workgroup by itself, 0.5 for
+// each of two workgroups' steps and 0.46 for each of three's (8,192 tokens: 263,000 steps of all heads
+// in 470 us).
+double deal(const std::vector<int32_t>& lens, int cus, std::vector<int32_t>* order) {
+  typedef std::pair<double, int> Load;
+  std::priority_queue<Load, std::vector<Load>, std::greater<Load>> open;
+  std::vector<std::vector<int32_t>> places(cus);
+  for (int c = 0; c < cus; ++c) open.push({0.0, c});
+  const int n = static_cast<int>(lens.size()), dealt = std::min(n, kPfPerCu * cus);
+  for (int i = 0; i < dealt; ++i) {
+    const Load at = open.top();
+    open.pop();
+    places[at.second].push_back(i);
+    if (static_cast<int>(places[at.second].size()) < kPfPerCu) open.push({at.first + lens[i], at.second});
+  }
+  if (order != nullptr) {
+    order->clear();
+    for (int round = 0; round < kPfPerCu; ++round)
+      for (int c = 0; c < cus; ++c)
+        if (round < static_cast<int>(places[c].size())) order->push_back(places[c][round]);
+    for (int i = dealt; i < n; ++i) order->push_back(i);
+  }
+  double most = 0;
+  std::priority_queue<double, std::vector<double>, std::greater<double>> times;
+  for (const auto& p : places) {
+    const double a = p.size() > 0 ? lens[p[0]] : 0, b = p.size() > 1 ? lens[p[1]] : 0, c = p.size() > 2 ? lens[p[2]] : 0;
+    times.push(0.46 * 3 * c + 0.5 * 2 * (b - c) + 0.66 * (a - b));
+    most = std::max(most, 0.46 * 3 * c + 0.5 * 2 * (b - c) + 0.66 * (a - b));
+  }
+  for (int i = dealt; i < n; ++i) {
+    const double now = times.top() + 0.46 * lens[i];
+    times.pop();
+    times.push(now);
+    most = std::max(most, now);
+  }
+  return most;
+}
+
+// Estimated us of a launch with the blocks cut at `piece` steps: every piece's rows are written and
+// read once in fp32 (about 5 TB/s) and merged by a launch of its own. The heads' workgroups go round
+// the XCDs, so a head has about 256 / num_kv_heads CUs.
+double estimate_us(const std::vector<int32_t>& steps, const std::vector<int32_t>& rows, int64_t piece, int num_kv_heads,
+                   std::vector<int32_t>& lens, int64_t& slots) {
+  lens.clear();
+  slots = 0;
+  double part_bytes = 0;
+  for (size_t i = 0; i < steps.size(); ++i) {
+    const int k = piece_count(steps[i], piece);
+    for (int j = 0; j < k; ++j) lens.push_back(static_cast<int32_t>((int64_t(steps[i]) + j) / k) + kPfStart);
+    if (k > 1) {
+      slots += k;
+      part_bytes += double(k) * rows[i] * num_kv_heads * 1024.0;
+    }
+  }
+  std::sort(lens.begin(), lens.end(), std::greater<int32_t>());
+  return deal(lens, std::max(1, 256 / num_kv_heads), nullptr) + (slots > 0 ? 6.0 + part_bytes / 5e6 : 0.0);
+}
+
+int prefill_launch(const aspire_prefill_args* a, const int32_t* units, int32_t num_units, const int32_t* merges,
+                   int32_t num_merges, int32_t num_slots, float* partials, int64_t partials_size, void* stream) {
   ASPIRE_CHECK_ARG(a != nullptr, "null argument");
   ASPIRE_CHECK_ARG(a->head_dim == kHeadDim && a->page_size == kPage, "head_dim 128 and page_size 16 only");
   const int bt = aspire_prefill_block_tokens(a->num_qo_heads, a->num_kv_heads);
@@ -493,8 +660,117 @@ extern "C" int aspire_prefill_run(const aspire_prefill_args* a, void* stream) {
   p.group = a->num_qo_heads / a->num_kv_heads;
   p.scale_log2 = a->sm_scale * 1.4426950408889634f;
   p.causal = a->causal;
-  hipLaunchKernelGGL(prefill_kernel, dim3(a->total_blocks * a->num_kv_heads), dim3(kPfThreads), 0,
-                     static_cast<hipStream_t>(stream), p);
+  p.units = reinterpret_cast<const int4*>(units);
+  const int64_t part_rows = int64_t(num_slots) * a->num_kv_heads * kPfBlockRows;
+  p.part_o = partials;
+  p.part_lse = partials + part_rows * kHeadDim;
+  if (units == nullptr)
+    num_units = a->total_blocks;
+  else
+    ASPIRE_CHECK_ARG(num_units > 0 && num_slots >= 0 && num_merges >= 0 && pf_al16(units) && pf_al16(merges) &&
+                         (num_slots == 0 || (partials && pf_al16(partials) && num_merges > 0 && merges &&
+                                             partials_size >= part_rows * (kHeadDim + 1))),
+                     "bad units, or partials smaller than slots * num_kv_heads * block rows * 129 floats");
+  ASPIRE_CHECK_ARG(int64_t(num_units) * a->num_kv_heads < (int64_t(1) << 31), "too many units");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(prefill_kernel, dim3(num_units * a->num_kv_heads), dim3(kPfThreads), 0, s, p);
+  if (units != nullptr && num_merges > 0)
+    hipLaunchKernelGGL(prefill_merge_kernel, dim3(num_merges * a->num_kv_heads * (kPfBlockRows / 16)), dim3(256), 0, s,
+                       p, reinterpret_cast<const int4*>(merges));
   ASPIRE_CHECK_LAUNCH();
+  return ASPIRE_OK;
+}
+
+}  // namespace
+}  // namespace aspire
+
+extern "C" int aspire_prefill_run(const aspire_prefill_args* a, void* stream) {
+  return aspire::prefill_launch(a, nullptr, 0, nullptr, 0, 0, nullptr, 0, stream);
+}
+
+extern "C" int aspire_prefill_run_units(const aspire_prefill_args* a, const int32_t* units, int32_t num_units,
+                                        const int32_t* merges, int32_t num_merges, int32_t num_slots, float* partials,
+                                        int64_t partials_size, void* stream) {
+  if (units == nullptr) return aspire::fail(ASPIRE_ERR_INVALID, "aspire_prefill_run_units: null units");
+  return aspire::prefill_launch(a, units, num_units, merges, num_merges, num_slots, partials, partials_size, stream);
+}
+
+extern "C" int aspire_prefill_plan(const int32_t* q_len, const int32_t* kv_len, int32_t num_rows, int32_t num_qo_heads,
+                                   int32_t num_kv_heads, int32_t causal, int64_t max_slots, int32_t* out, int64_t out_size,
+                                   int32_t* num_units, int32_t* num_merges, int32_t* num_slots) {
+  using namespace aspire;
+  const int bt = aspire_prefill_block_tokens(num_qo_heads, num_kv_heads);
+  ASPIRE_CHECK_ARG(bt > 0 && num_rows >= 0 && (num_rows == 0 || (q_len && kv_len)) && num_units && num_merges && num_slots,
+                   "bad arguments");
+  try {
+    std::vector<int32_t> steps, rows_of;  // of every query block, in block order
+    int64_t total = 0;
+    for (int b = 0; b < num_rows; ++b) {
+      for (int64_t t0 = 0; t0 < q_len[b]; t0 += bt) {
+        const int64_t end = std::min<int64_t>(t0 + bt, q_len[b]);
+        const int64_t keys = causal ? std::min<int64_t>(int64_t(kv_len[b]) - q_len[b] + end, kv_len[b]) : kv_len[b];
+        const int64_t pages = keys > 0 ? (keys + kPage - 1) / kPage : 0;
+        steps.push_back(static_cast<int32_t>((pages + 1) / 2));
+        rows_of.push_back(static_cast<int32_t>(end - t0) * (num_qo_heads / num_kv_heads));
+        total += steps.back();
+      }
+    }
+    const int n = static_cast<int>(steps.size());
+    // Whole blocks, or pieces from 2.5 down to 0.5 times an even share of the chip's 768 workgroup
+    // slots (16 steps at least), whichever the estimate likes best. Whole -> cut, us: 64 tokens over
+    // 16,000 332 -> 38, 5 rows of 17 to 700 tokens over 300 to 8,192 196 -> 158, 300 over 8,000 171 -> 60.
+    int64_t piece = int64_t(1) << 40, slots_of;
+    const int32_t longest = n > 0 ? *std::max_element(steps.begin(), steps.end()) : 0;
+    int64_t last = 0;
+    std::vector<int32_t> lens;
+    double best = estimate_us(steps, rows_of, piece, num_kv_heads, lens, slots_of);
+    for (double f = 2.5; f >= 0.5; f -= 0.25) {
+      const int64_t cut = std::max<int64_t>(16, int64_t(f * double(total) * num_kv_heads / 768));
+      if (piece_count(longest, cut) == 1 || (f < 2.5 && cut == last)) continue;  // whole blocks, or the same pieces again
+      last = cut;
+      const double us = estimate_us(steps, rows_of, cut, num_kv_heads, lens, slots_of);
+      if (us < best && slots_of <= max_slots) {
+        best = us;
+        piece = cut;
+      }
+    }
+    struct Unit {
+      int32_t blk, begin, end, slot, len;
+    };
+    std::vector<Unit> units;
+    std::vector<int32_t> merges;
+    int32_t slots = 0;
+    for (int i = n - 1; i >= 0; --i) {
+      const int32_t s = steps[i];
+      const int32_t k = piece_count(s, piece);
+      if (k > 1) merges.insert(merges.end(), {i, slots, k, 0});
+      for (int32_t j = 0; j < k; ++j) {
+        const int32_t at = static_cast<int32_t>(int64_t(s) * j / k), to = static_cast<int32_t>(int64_t(s) * (j + 1) / k);
+        units.push_back(Unit{i, at, j + 1 == k ? 0x7fffffff : to, k > 1 ? slots++ : -1, to - at});
+      }
+    }
+    std::stable_sort(units.begin(), units.end(), [](const Unit& x, const Unit& y) { return x.len > y.len; });
+    *num_units = static_cast<int32_t>(units.size());
+    *num_merges = static_cast<int32_t>(merges.size() / 4);
+    *num_slots = slots;
+    if (out != nullptr) {
+      ASPIRE_CHECK_ARG(out_size >= int64_t(units.size()) * 4 + int64_t(merges.size()), "out is too small");
+      lens.clear();
+      for (const Unit& u : units) lens.push_back(u.len);
+      std::vector<int32_t> order;
+      deal(lens, std::max(1, 256 / num_kv_heads), &order);
+      for (int32_t i : order) {
+        const Unit& u = units[i];
+        *out++ = u.blk;
+        *out++ = u.begin;
+        *out++ = u.end;
+        *out++ = u.slot;
+      }
+      std::copy(merges.begin(), merges.end(), out);
+    }
+  } catch (const std::exception& e) {
+    set_error("aspire_prefill_plan: %s", e.what());
+    return ASPIRE_ERR_CAPACITY;
+  }
   return ASPIRE_OK;
 }

@@ -497,6 +497,19 @@ int aspire_prefill_block_tokens(int32_t num_qo_heads, int32_t num_kv_heads);
 
 int aspire_prefill_run(const aspire_prefill_args* args, void* stream);
 
+/* The same with the blocks' keys cut into pieces, for batches whose blocks are too few or too uneven to
+ * fill the chip. aspire_prefill_plan (host only, host arrays) writes num_units x 4 int32 units and then
+ * num_merges x 4 int32 merges into out (NULL: the counts alone); it cuts into at most max_slots pieces.
+ * The two tables go to the device; partials holds num_slots * num_kv_heads * block rows * 129 floats,
+ * block rows = block_tokens * num_qo_heads / num_kv_heads. A table stays valid, if less even, when the
+ * rows' kv lengths change. */
+int aspire_prefill_plan(const int32_t* q_len, const int32_t* kv_len, int32_t num_rows, int32_t num_qo_heads,
+                        int32_t num_kv_heads, int32_t causal, int64_t max_slots, int32_t* out, int64_t out_size,
+                        int32_t* num_units, int32_t* num_merges, int32_t* num_slots);
+int aspire_prefill_run_units(const aspire_prefill_args* args, const int32_t* units, int32_t num_units,
+                             const int32_t* merges, int32_t num_merges, int32_t num_slots, float* partials,
+                             int64_t partials_size, void* stream);
+
 /* ------------------------------------------------------ (f4) sampling
  * Token sampling and speculative verification. One workgroup per row or request; the
  * uniforms of every draw are explicit device inputs (the Python layer draws them with

@@ -195,3 +195,78 @@ def test_prefill_wrapper_graph_replays_later_plans(gpu, use_cuda_graph):
         out = w.run(q_buf, step.cache)
         torch.cuda.synchronize()
         attn_close(out[:T], ref[:T])
+
+
+def _pieces(step, bt, piece, causal):
+    """Every query block of ``step`` cut at ``piece`` steps: (units, merges, slots) as aspire_prefill_plan
+    writes them, in any order."""
+    units, merges, slots, blk = [], [], 0, 0
+    for q, k in zip(step.q_len, step.ctx_len):
+        for t0 in range(0, int(q), bt):
+            keys = int(min(k - q + min(t0 + bt, q), k) if causal else k)
+            n = max(-(-(-(-keys // 16) + 1) // 2 // piece), 1) if keys > 0 else 1
+            if n > 1:
+                merges.append((blk, slots, n, 0))
+            for j in range(n):
+                units.append((blk, j * piece, 0x7FFFFFFF if j == n - 1 else (j + 1) * piece, slots if n > 1 else -1))
+                slots += n > 1
+            blk += 1
+    to = lambda x: torch.tensor(x, dtype=torch.int32).view(-1, 4)
+    return to(units[::-1]), to(merges), slots
+
+
+@pytest.mark.parametrize("hq,hkv,ctx,q_len", [
+    (32, 8, [257, 1001, 40, 900], [257, 33, 1, 129]), (8, 8, [300, 700], [300, 200]), (64, 2, [513, 70], [20, 70])])
+@pytest.mark.parametrize("piece", [1, 2, 5])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_cut_into_pieces_matches_oracle(gpu, monkeypatch, hq, hkv, ctx, q_len, piece, causal):
+    """Blocks cut at 1, 2 and 5 steps of 32 keys, so that a piece holds keys that some of its rows, or none
+    of a row's keys, see; rows ending mid-page and mid-step, stale tail slots of NaN keys and inf values."""
+    say("prefill pieces", hq, hkv, piece, causal)
+    step = build_step(hq=hq, hkv=hkv, ctx_len=ctx, q_len=q_len, is_draft=[0] * len(ctx), draft_budget=0, seed=40,
+                      device=gpu)
+    cache = step.cache.clone()
+    table = step.block_table.cpu().numpy()
+    for b, n in enumerate(ctx):
+        if n % PAGE:
+            page = int(table[b, n // PAGE])
+            cache[page, 0, n % PAGE :] = float("nan")
+            cache[page, 1, n % PAGE :] = float("inf")
+    seen = {}
+
+    def plan_units(ql, kl, bt, *args):
+        u, m, s = _pieces(step, bt, piece, causal)
+        seen["slots"] = s
+        return u, m, s
+
+    monkeypatch.setattr(BatchPrefillWithPagedKVCacheWrapper, "_plan_units", staticmethod(plan_units))
+    w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(1, device=gpu), "NHD")
+    w.plan(step.qo_indptr[:-1], step.kv_indptr[:-1], step.kv_indices, step.last_page_len[:-1], hq, hkv, 128, PAGE,
+           causal=causal)
+    assert seen["slots"] > len(ctx)
+    out, lse = w.run(step.q, cache, return_lse=True)
+    ref_out, ref_lse = paged_attention(step.q.cpu(), step.cache.cpu(), step.qo_indptr_host, step.kv_indptr_host,
+                                       step.kv_indices.cpu(), step.kv_len_host, num_kv_heads=hkv, causal=causal)
+    T = step.total_tokens
+    attn_close(out[:T], ref_out[:T])
+    assert (lse[:T].cpu() - ref_lse[:T]).abs().max() < 2e-3
+
+
+def test_prefill_long_prefix_is_cut_and_matches_whole_blocks(gpu, monkeypatch):
+    """A short chunk over a long prefix, as the plan cuts it, against the same launch with whole blocks."""
+    say("prefill long prefix")
+    step = build_step(hq=32, hkv=8, ctx_len=[12001, 5000], q_len=[65, 7], is_draft=[0, 0], draft_budget=0, seed=41, device=gpu)
+    args = (step.qo_indptr[:-1], step.kv_indptr[:-1], step.kv_indices, step.last_page_len[:-1], 32, 8, 128, PAGE)
+    outs = []
+    for cut in (True, False):
+        if not cut:
+            whole = [(blk, 0, 0x7FFFFFFF, -1) for blk in range(4)]
+            monkeypatch.setattr(BatchPrefillWithPagedKVCacheWrapper, "_plan_units", staticmethod(
+                lambda *a: (torch.tensor(whole, dtype=torch.int32), torch.empty(0, 4, dtype=torch.int32), 0)))
+        w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(1, device=gpu), "NHD")
+        w.plan(*args, causal=True)
+        assert (w._pf["slots"] > 0) == cut
+        outs.append(w.run(step.q, step.cache, return_lse=True))
+    (a, la), (b, lb) = outs
+    attn_close(a, b)
+    assert (la - lb).abs().max() < 1e-4

@@ -353,3 +353,58 @@ def test_merge_row_ranges_lone_long_row():
     _, merges = decode(lay, buf, info)
     long = merges[merges[:, 5] == 36]
     assert len(long) and (long[:, 4] > 16).all() and (long[:, 7] == 12).all()
+
+
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (8, 8), (64, 2)])
+@pytest.mark.parametrize("causal", [1, 0])
+@pytest.mark.parametrize("q_len,kv_len,max_slots", [
+    ([64], [16064], 500), ([17, 0, 700, 300], [8000, 0, 9000, 300], 500), ([64], [16064], 20), ([8192], [8192], 500),
+    ([1], [1], 500), ([0], [0], 500), ([5], [3], 500), ([300] * 40, [5000] * 40, 500)])
+def test_prefill_units_cover_every_step_once(hq, hkv, causal, q_len, kv_len, max_slots):
+    """Every query block's steps [0, steps) are in exactly one piece each, the last piece open-ended; the
+    partial slots of a cut block are consecutive and belong to it alone; no more slots than allowed."""
+    import ctypes
+
+    import torch
+
+    from aspire_amd import _lib
+
+    lib = _lib.lib()
+    ql, kl = torch.tensor(q_len, dtype=torch.int32), torch.tensor(kv_len, dtype=torch.int32)
+    n = [ctypes.c_int32() for _ in range(3)]
+
+    def plan(out, size):
+        rc = lib.aspire_prefill_plan(_lib.ptr(ql), _lib.ptr(kl), len(q_len), hq, hkv, causal, max_slots, _lib.ptr(out), size,
+                                     *(ctypes.byref(x) for x in n))
+        return rc
+
+    assert plan(None, 0) == 0
+    units, merges, slots = (x.value for x in n)
+    out = torch.full((units + merges + 1, 4), -7, dtype=torch.int32)
+    assert plan(out, 4 * (units + merges)) == 0 and (out[-1] == -7).all()
+    if units:
+        assert plan(out, 4 * (units + merges) - 1) == _lib.ASPIRE_ERR_INVALID  # nothing written past a short buffer
+    bt = lib.aspire_prefill_block_tokens(hq, hkv)
+    steps = []
+    for q, k in zip(q_len, kv_len):
+        for t0 in range(0, q, bt):
+            keys = min(k - q + min(t0 + bt, q), k) if causal else k
+            steps.append((max(-(-keys // 16), 0) + 1) // 2)
+    assert slots <= max_slots
+    pieces = {}
+    for blk, begin, end, slot in out[:units].tolist():
+        pieces.setdefault(blk, []).append((begin, end, slot))
+    assert sorted(pieces) == list(range(len(steps)))
+    merge_of = {blk: (first, count) for blk, first, count, _ in out[units : units + merges].tolist()}
+    used = []
+    for blk, got in pieces.items():
+        got.sort()
+        assert got[0][0] == 0 and got[-1][1] == 0x7FFFFFFF
+        assert all(a[1] == b[0] and a[0] < a[1] for a, b in zip(got, got[1:])) and got[-1][0] <= max(steps[blk] - 1, 0)
+        if len(got) == 1:
+            assert got[0][2] == -1 and blk not in merge_of
+        else:
+            first, count = merge_of[blk]
+            assert count == len(got) and [p[2] for p in got] == list(range(first, first + count))
+            used += [p[2] for p in got]
+    assert sorted(used) == list(range(slots)) and len(merge_of) == merges
