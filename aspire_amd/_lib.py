@@ -270,19 +270,27 @@ def check(rc: int, what: str) -> None:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    # a plain address: every parameter it goes to is declared c_void_p
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(t: torch.Tensor):
-    """The current HIP stream of ``t``'s device as a ctypes pointer."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """The address of the current HIP stream of ``t``'s device. ``t`` is a GPU tensor (the
+    callers have checked it), so torch is initialised; the raw getter spares the Stream object
+    that ``torch.cuda.current_stream`` builds (1.6 against 0.2 us, in every call of the package)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_cuda(*tensors: torch.Tensor, what: str) -> None:
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(f"{what}: tensors must be on a ROCm GPU (got {t.device}); "
                                "there is no CPU implementation")
+
+
+def dense(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """``t.to(dtype).contiguous()``, without the two calls where ``t`` is that already."""
+    return t if t.dtype == dtype and t.is_contiguous() else t.to(dtype).contiguous()
 
 
 def build_info() -> str:

@@ -270,6 +270,10 @@ class HolisticAttentionWrapper:
 
         self._plan_host_lens = (qo, kvl)
         self._plan_info = info
+        # what an eager run of this plan launches (see run)
+        self._plan_class_mask = sum(1 << c for c in range(3) if info.num_items[c] > 0)
+        self._plan_merge = 1 if info.num_merge > 0 else 0
+        self._plan_nt = 1 if info.total_pages <= SHORT_PLAN_PAGES_PER_WAVE * self._layout.num_waves else 0
         self._plan_tokens = int(qo[: batch + 1].max()) if batch else 0
         # rows that can write dump entries / page scores: queries and at least one page
         if per_head_lists:
@@ -311,38 +315,50 @@ class HolisticAttentionWrapper:
         """
         if not self._planned:
             raise RuntimeError("run() requires plan() or plan_host() first")
-        k_cache, v_cache = _unpack_paged_kv_cache(paged_kv_cache, self._kv_layout)
+        if isinstance(paged_kv_cache, torch.Tensor) and paged_kv_cache.dim() == 5 and paged_kv_cache.shape[1] == 2:
+            # one tensor: K and V share everything but their offset, so the two views (3 us of
+            # host time) are not built
+            k_cache = v_cache = paged_kv_cache
+            _, _, page_size, num_kv_heads, _ = paged_kv_cache.shape
+            cache_st_p, kv_off, cache_st_t, cache_st_h, cache_st_d = paged_kv_cache.stride()
+            kv_off *= paged_kv_cache.element_size()
+        else:
+            k_cache, v_cache = _unpack_paged_kv_cache(paged_kv_cache, self._kv_layout)
+            page_size, num_kv_heads = k_cache.shape[1:3]
+            cache_st_p, cache_st_t, cache_st_h, cache_st_d = k_cache.stride()[:4]
+            kv_off = v_cache.data_ptr() - k_cache.data_ptr()
         _lib.require_cuda(q, k_cache, v_cache, what="HolisticAttentionWrapper.run")
-        if q.dim() != 3 or q.shape[2] != 128 or q.stride(2) != 1:
+        q_shape, q_st = q.shape, q.stride()
+        if len(q_shape) != 3 or q_shape[2] != 128 or q_st[2] != 1:
             raise ValueError("q must be [T, num_qo_heads, 128] with a contiguous head dimension")
-        if q.shape[1] != self._num_qo_heads:
-            raise ValueError(f"q has {q.shape[1]} heads, plan has {self._num_qo_heads}")
+        if q_shape[1] != self._num_qo_heads:
+            raise ValueError(f"q has {q_shape[1]} heads, plan has {self._num_qo_heads}")
         if q.dtype != torch.bfloat16 or k_cache.dtype != torch.bfloat16:
             raise ValueError("the HIP attention kernel computes in bf16 (q and kv_cache)")
-        if k_cache.stride() != v_cache.stride() or k_cache.stride(3) != 1:
+        if k_cache.stride() != v_cache.stride() or cache_st_d != 1:
             raise ValueError("k and v caches must share strides with a contiguous head dimension")
-        if k_cache.shape[1] != self._page_size or k_cache.shape[2] != self._num_kv_heads:
+        if page_size != self._page_size or num_kv_heads != self._num_kv_heads:
             raise ValueError("kv_cache page size / kv heads disagree with the plan")
-        if q.shape[0] < self._plan_tokens:
-            raise ValueError(f"q has {q.shape[0]} tokens, the plan addresses {self._plan_tokens}")
+        if q_shape[0] < self._plan_tokens:
+            raise ValueError(f"q has {q_shape[0]} tokens, the plan addresses {self._plan_tokens}")
         if out is None:
-            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        if out.shape != q.shape or out.stride(2) != 1 or out.dtype != q.dtype:
+            out = torch.empty(q_shape, dtype=q.dtype, device=q.device)
+        out_st = out.stride()
+        if out.shape != q_shape or out_st[2] != 1 or out.dtype != q.dtype:
             raise ValueError("out must match q's shape and dtype with a contiguous head dimension")
-        lse = torch.empty(q.shape[0], q.shape[1], device=q.device, dtype=torch.float32)
-        sm_scale = self._sm_scale if self._sm_scale is not None else 1.0 / math.sqrt(q.shape[2])
+        lse = torch.empty(q_shape[0], q_shape[1], device=q.device, dtype=torch.float32)
+        sm_scale = self._sm_scale if self._sm_scale is not None else 1.0 / math.sqrt(q_shape[2])
         elem = k_cache.element_size()
-        kv_off = (v_cache.data_ptr() - k_cache.data_ptr())
         if kv_off % elem:
             raise ValueError("v_cache is not element-aligned with k_cache")
 
         a = _lib.AttentionArgs()
-        a.q, a.q_stride_t, a.q_stride_h = q.data_ptr(), q.stride(0), q.stride(1)
+        a.q, a.q_stride_t, a.q_stride_h = q.data_ptr(), q_st[0], q_st[1]
         a.kv_cache = k_cache.data_ptr()
-        a.cache_stride_p, a.cache_stride_kv = k_cache.stride(0), kv_off // elem
-        a.cache_stride_t, a.cache_stride_h = k_cache.stride(1), k_cache.stride(2)
+        a.cache_stride_p, a.cache_stride_kv = cache_st_p, kv_off // elem
+        a.cache_stride_t, a.cache_stride_h = cache_st_t, cache_st_h
         a.kv_indices = self._kv_indices.data_ptr()
-        a.out, a.out_stride_t, a.out_stride_h = out.data_ptr(), out.stride(0), out.stride(1)
+        a.out, a.out_stride_t, a.out_stride_h = out.data_ptr(), out_st[0], out_st[1]
         a.lse = lse.data_ptr()
         a.plan_dev = self._int_workspace.data_ptr()
         a.float_ws = self._float_workspace.data_ptr()
@@ -353,11 +369,10 @@ class HolisticAttentionWrapper:
         if self._use_cuda_graph or torch.cuda.is_current_stream_capturing():
             a.class_mask, a.launch_merge = 7, 1
         else:
-            a.class_mask = sum(1 << c for c in range(3) if info.num_items[c] > 0)
-            a.launch_merge = 1 if info.num_merge > 0 else 0
+            a.class_mask, a.launch_merge = self._plan_class_mask, self._plan_merge
         # short plans store their split-KV partials non-temporally (a graph keeps the choice
         # of the plan it was captured with; either is correct for any plan)
-        a.partial_nt = 1 if info.total_pages <= SHORT_PLAN_PAGES_PER_WAVE * self._layout.num_waves else 0
+        a.partial_nt = self._plan_nt
         keep_alive = [q, out, lse]
         wants_dump = self._has_jit and self._dump is not None and self._dump.kind != "noop"
         if (wants_dump or page_scores is not None) and info.split_rows > 0:

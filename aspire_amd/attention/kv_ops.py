@@ -37,11 +37,12 @@ def paged_kv_append(k, v, kv_append_indptr, kv_cache, kv_page_indices, kv_page_i
     _lib.require_cuda(k, v, kv_cache, kv_append_indptr, kv_page_indices, what="update_kv_padded")
     head_dim = k.shape[2]
     num_heads = k.shape[1]
-    if k.stride(-1) != 1 or v.stride(-1) != 1:
+    ks, vs, cs = k.stride(), v.stride(), kv_cache.stride()
+    if ks[-1] != 1 or vs[-1] != 1:
         raise ValueError("update_kv_padded requires contiguous k/v head dimensions")
-    if k.stride(1) != head_dim or v.stride(1) != head_dim:
+    if ks[1] != head_dim or vs[1] != head_dim:
         raise ValueError("update_kv_padded requires contiguous k/v heads")
-    if kv_cache.stride(-1) != 1:
+    if cs[-1] != 1:
         raise ValueError("update_kv_padded requires a contiguous cache head dimension")
     if k.dtype != kv_cache.dtype or v.dtype != kv_cache.dtype or kv_cache.element_size() != 2:
         raise ValueError("k, v and kv_cache must share a 16-bit dtype")
@@ -52,9 +53,9 @@ def paged_kv_append(k, v, kv_append_indptr, kv_cache, kv_page_indices, kv_page_i
                       _i32(kv_last_page_len))
     L = _lib.lib()
     rc = L.aspire_paged_kv_append(
-        _lib.ptr(k), _lib.ptr(v), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
+        _lib.ptr(k), _lib.ptr(v), ks[0], ks[1], vs[0], vs[1],
         _lib.ptr(ai), _lib.ptr(pi), _lib.ptr(pp), _lib.ptr(lp), num_seq,
-        _lib.ptr(kv_cache), kv_cache.stride(0), kv_cache.stride(1), kv_cache.stride(2), kv_cache.stride(3),
+        _lib.ptr(kv_cache), cs[0], cs[1], cs[2], cs[3],
         total_tokens, num_heads, head_dim, int(page_size), _lib.stream_of(k),
     )
     _lib.check(rc, "update_kv_padded")

@@ -33,16 +33,17 @@ def local_topk_candidates(logits: torch.Tensor, top_k: int, vocab_start: int = 0
     if logits.dtype != torch.bfloat16:
         raise ValueError("the HIP top-k kernel reads bf16 logits")
     lead = logits.shape[:-1]
-    x = logits.reshape(-1, logits.shape[-1])
+    x = logits if logits.dim() == 2 else logits.reshape(-1, logits.shape[-1])
     if x.stride(-1) != 1:
         x = x.contiguous()
     rows, vocab = x.shape
-    values = torch.empty(rows, top_k, dtype=logits.dtype, device=logits.device)
-    ids = torch.empty(rows, top_k, dtype=torch.int64, device=logits.device)
+    dev = logits.device
+    values = torch.empty(*lead, top_k, dtype=logits.dtype, device=dev)
+    ids = torch.empty(*lead, top_k, dtype=torch.int64, device=dev)
     rc = _lib.lib().aspire_topk_candidates(_lib.ptr(x), x.stride(0), rows, vocab, top_k, int(vocab_start),
                                            _lib.ptr(values), _lib.ptr(ids), _lib.stream_of(logits))
     _lib.check(rc, "local_topk_candidates")
-    return values.view(*lead, top_k), ids.view(*lead, top_k)
+    return values, ids
 
 
 def merge_topk_candidates(values: torch.Tensor, indices: torch.Tensor, top_k: int):
@@ -75,12 +76,9 @@ def verify_topk_speculation(draft_probs: torch.Tensor, draft_ids: torch.Tensor, 
     if draft_counts.shape != (requests,):
         raise ValueError("draft_counts must hold one count per request")
     dev = draft_probs.device
-    dp = draft_probs.to(torch.float32).contiguous()
-    tp = target_probs.to(torch.float32).contiguous()
-    di = draft_ids.to(torch.int64).contiguous()
-    ti = target_ids.to(torch.int64).contiguous()
-    tok = draft_tokens.to(torch.int32).contiguous()
-    cnt = draft_counts.to(torch.int32).contiguous()
+    dp, tp = _lib.dense(draft_probs, torch.float32), _lib.dense(target_probs, torch.float32)
+    di, ti = _lib.dense(draft_ids, torch.int64), _lib.dense(target_ids, torch.int64)
+    tok, cnt = _lib.dense(draft_tokens, torch.int32), _lib.dense(draft_counts, torch.int32)
     if uniforms is None:
         uniforms = torch.rand(requests, max_draft + 1, device=dev, generator=generator)
     elif uniforms.shape != (requests, max_draft + 1) or uniforms.dtype != torch.float32:

@@ -54,17 +54,17 @@ class LogitsPipe:
         if values.dtype not in (torch.bfloat16, torch.float32):
             raise ValueError("values must be bf16 or fp32")
         shape = values.shape
-        v = values.reshape(-1, shape[-1])
+        v = values if values.dim() == 2 else values.reshape(-1, shape[-1])
         if v.stride(-1) != 1:
             v = v.contiguous()
         rows, width = v.shape
-        probs = torch.empty(rows, width, dtype=torch.float32, device=values.device)
+        probs = torch.empty(shape, dtype=torch.float32, device=values.device)
         rc = _lib.lib().aspire_logits_pipe(
             _lib.ptr(v), 1 if v.dtype == torch.float32 else 0, v.stride(0), rows, width,
             float(temperature) if self._temperature else 0.0, float(top_p) if self._top_p else 0.0,
-            _lib.ptr(probs), probs.stride(0), _lib.stream_of(values))
+            _lib.ptr(probs), width, _lib.stream_of(values))
         _lib.check(rc, "LogitsPipe")
-        return probs.view(shape)
+        return probs
 
 
 def define_logit_process_op(pipe: LogitsPipe, kwargs: dict):

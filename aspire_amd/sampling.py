@@ -67,9 +67,8 @@ def chain_speculative_sampling(draft_probs: torch.Tensor, draft_token_ids: torch
     B, D, V = draft_probs.shape
     if target_probs.shape != (B, D + 1, V) or draft_token_ids.shape != (B, D):
         raise ValueError("shapes disagree: target_probs must be [B, D + 1, V], draft_token_ids [B, D]")
-    dp = draft_probs.to(torch.float32).contiguous()
-    tp = target_probs.to(torch.float32).contiguous()
-    ids = draft_token_ids.to(torch.int32).contiguous()
+    dp, tp = _lib.dense(draft_probs, torch.float32), _lib.dense(target_probs, torch.float32)
+    ids = _lib.dense(draft_token_ids, torch.int32)
     dev = dp.device
     out = torch.empty(B, D + 1, dtype=torch.int32, device=dev)
     acc = torch.empty(B, dtype=torch.int32, device=dev)

@@ -447,3 +447,29 @@ def test_partial_store_kinds_are_bitwise_identical(gpu, monkeypatch, ctx, q_len,
     assert torch.equal(l0[:T], l1[:T])
     ref_out, ref_lse = oracle(step, step.cache)
     check_rows(step, o1, l1, ref_out, ref_lse)
+
+
+@pytest.mark.parametrize("form", ["strided", "views", "separate"])
+def test_cache_forms_read_the_same_values(gpu, form):
+    """One tensor, a strided one, its two views and two tensors of their own hold the same K and V."""
+    say("cache forms", form)
+    step = build_step(hq=16, hkv=8, ctx_len=[300, 77, 1030], q_len=[1, 5, 2], is_draft=[1, 0, 0], draft_budget=9, seed=4,
+                      device=gpu, bucket_tokens=8)
+    w = make_wrapper(gpu)
+    plan(w, step)
+    want, want_lse = w.run(step.q, step.cache, return_lse=True)
+    if form == "strided":  # the heads of a wider cache
+        wide = torch.zeros(*step.cache.shape[:3], 12, 128, dtype=torch.bfloat16, device=gpu)
+        wide[:, :, :, 2:10] = step.cache
+        cache = wide[:, :, :, 2:10]
+    elif form == "views":
+        cache = (step.cache[:, 0], step.cache[:, 1])
+    else:
+        cache = (step.cache[:, 0].contiguous(), step.cache[:, 1].contiguous())
+    got, lse = w.run(step.q, cache, return_lse=True)
+    T = step.total_tokens
+    # the strided form may take another load path; all compute the same products in the same order per row
+    attn_close(got[:T], want[:T])
+    assert (lse[:T] - want_lse[:T]).abs().max().item() < 2e-3
+    with pytest.raises(ValueError, match="contiguous head dimension"):
+        w.run(step.q, step.cache.transpose(3, 4).contiguous().transpose(3, 4))
