@@ -28,6 +28,19 @@ namespace aspire {
 namespace {
 
 constexpr int kMinPagesPerWave = 8;
+// Short plans (fewer than kMinPagesPerWave pages for every slot) are bound by latency, not by
+// bandwidth: a wave spends 3.7 us up to its first page (plan, item, page id and K/V in series),
+// 1.0 us on each page (the chain from the LDS read to P.V), about 2 us more on a second item,
+// and the merge 1.5 us on each round of partials. Their rows are therefore cut by themselves,
+// one piece to a slot, at the piece length whose modelled time is least: its pages, plus, where
+// a row is cut, the merge's launch and rounds and the partials' traffic (written and read at
+// 2 TB/s). Attention and merge with K/V read from HBM, against streams of 8 pages that cross
+// rows (16 query / 8 kv heads): 4 rows of 1024 keys x 5 queries 17.3 -> 13.9 us, of 2048
+// 19.1 -> 16.8, 32 rows of 300 19.8 -> 15.6, 8 draft rows of 64 pages 17.5 -> 14.7; 16 rows
+// of 512 at 32/4 heads 24.9 -> 16.6. Where shorter pieces lose (4 rows of 4096 at 32/4 heads:
+// 26.0 us at 4 pages, the partials) the model stays at 8 (22.8 -> 23.0).
+constexpr int kShortPieceMin = 3, kShortPieceMax = 12;
+constexpr float kMergeLaunchUs = 3.5f, kMergeRoundUs = 1.5f, kPartialBytesPerUs = 2e6f;
 // Stream-K cost units of one page-head, in quarters: an item staged for the workgroup's heads
 // (32 for 2- and 3-tile items, 33 for 1-tile items) and an item reading its own head's list
 // (direct: 48). Per-wave finish times of config-4 launches (fitted per class) showed 1-tile
@@ -233,6 +246,34 @@ int plan_core(const aspire_plan_layout* layout, const int32_t* qo_indptr, const 
   const int64_t slots = W / hpu;
   // Slots actually used: enough that each streams >= kMinPagesPerWave pages.
   int64_t s_eff = std::max<int64_t>(1, std::min<int64_t>(slots, T_pages / kMinPagesPerWave));
+  // Short plans: the pages per piece (0: stream-K).
+  auto pieces_at = [&](const Segment& s, int m) -> int64_t {  // a direct page counts 3/2 (its cost)
+    return s.direct ? (int64_t(s.npages) * 3 + 2 * m - 1) / (2 * m) : (int64_t(s.npages) + m - 1) / m;
+  };
+  int piece_pages = 0;
+  if (T_pages / kMinPagesPerWave < slots) {
+    float best = 0.f;
+    for (int m = kShortPieceMin; m <= kShortPieceMax; ++m) {
+      int64_t used = 0, rows = 0, rounds = 0;
+      for (int c = 0; c < 3; ++c)
+        for (const auto& s : sc.segs[c]) {
+          const int64_t n = pieces_at(s, m);
+          used += n;
+          if (n < 2) continue;
+          rows += n * s.rows;
+          rounds = std::max<int64_t>(rounds, (n + 4 * kMergeChunk - 1) / (4 * kMergeChunk));
+        }
+      if (used > slots || rows * hpu > L.partial_rows_cap) continue;
+      float us = float(m);
+      if (rows > 0)
+        us += kMergeLaunchUs + kMergeRoundUs * float(rounds) +
+              float(rows * hpu) * float(L.head_dim * sizeof(float)) / kPartialBytesPerUs;
+      if (piece_pages == 0 || us < best) {
+        best = us;
+        piece_pages = m;
+      }
+    }
+  }
   // Shrink until the split pieces' partial rows fit the float workspace.
   for (;;) {
     for (auto& v : sc.citems) v.clear();
@@ -240,6 +281,7 @@ int plan_core(const aspire_plan_layout* layout, const int32_t* qo_indptr, const 
     int64_t pr = 0;
     int64_t seg_off = 0;
     int zero_rr = 0;
+    int64_t next_slot = 0;
     for (int c = 0; c < 3; ++c) {
       auto& out = sc.citems[c];
       for (const auto& s : sc.segs[c]) {
@@ -265,12 +307,18 @@ int plan_core(const aspire_plan_layout* layout, const int32_t* qo_indptr, const 
         auto first_page_at = [&](int64_t x) {  // first page whose position is >= x
           return x <= a ? int64_t(0) : std::min<int64_t>(s.npages, (x - a + wt - 1) / wt);
         };
-        const int64_t j_lo = slot_of(a), j_hi = slot_of(e - wt);
         sc.pieces.clear();
-        for (int64_t j = j_lo; j <= j_hi; ++j) {
-          const int64_t pb = first_page_at((j * T) / s_eff);
-          const int64_t pe = j == j_hi ? s.npages : first_page_at(((j + 1) * T) / s_eff);
-          if (pe > pb) sc.pieces.push_back({j, pb, pe});
+        if (piece_pages > 0) {
+          const int64_t n = pieces_at(s, piece_pages);
+          for (int64_t k = 0; k < n; ++k)
+            sc.pieces.push_back({next_slot++, k * s.npages / n, (k + 1) * s.npages / n});
+        } else {
+          const int64_t j_lo = slot_of(a), j_hi = slot_of(e - wt);
+          for (int64_t j = j_lo; j <= j_hi; ++j) {
+            const int64_t pb = first_page_at((j * T) / s_eff);
+            const int64_t pe = j == j_hi ? s.npages : first_page_at(((j + 1) * T) / s_eff);
+            if (pe > pb) sc.pieces.push_back({j, pb, pe});
+          }
         }
         const int pieces = static_cast<int>(sc.pieces.size());
         // partial rows: head gg's pieces are contiguous, first[gg] + k * rows

@@ -355,6 +355,36 @@ def test_merge_row_ranges_lone_long_row():
     assert len(long) and (long[:, 4] > 16).all() and (long[:, 7] == 12).all()
 
 
+@pytest.mark.parametrize("hq,hkv,q_len,kv_len,float_ws", [
+    (16, 8, [1, 1, 5, 5], [1024, 1000, 4096, 4090], 384 << 20),
+    (32, 8, [5, 0, 12, 1], [16, 300, 0, 513], 384 << 20),      # no queries, no keys, one page, a 3-tile row
+    (16, 2, [1, 3], [5000, 77], 384 << 20),                    # 2 kv heads: not head-aligned
+    (32, 4, [9] * 16, [512] * 16, 384 << 20),
+    (16, 8, [1] * 128, [17] * 128, 384 << 20),                 # as many rows as slots
+    (16, 8, [5] * 4, [8 * 16 * 128 // 4 - 16] * 4, 384 << 20),  # the longest short plan
+    (16, 8, [5], [4096], 2 << 20),                             # little room for partials
+])
+@pytest.mark.parametrize("per_head", [False, True])
+def test_short_plans_cut_rows_by_themselves(hq, hkv, q_len, kv_len, float_ws, per_head):
+    lay = layout(waves_per_cu=4, float_ws=float_ws)
+    reps = hkv if per_head else 1
+    qo, kvl = np.cumsum([0] + q_len), np.repeat(kv_len, reps)
+    kvp = np.cumsum(np.concatenate([[0], (kvl + 15) // 16]))
+    buf, info = plan(lay, qo, kvp, kvl, hq, hkv, per_head=per_head)
+    check_cover(lay, buf, info, qo, kvp, kvl, hq, hkv, per_head=per_head)
+    items = [(ip, it[it[:, 5] > it[:, 4]], it) for ip, it in decode(lay, buf, info)[0]]
+    held = np.zeros(lay.num_waves, dtype=int)
+    for ip, _, it in items:
+        for w in range(lay.num_waves):
+            held[w] += int((it[ip[w] : ip[w + 1], 5] > it[ip[w] : ip[w + 1], 4]).sum())
+    assert held.max() <= 1, "a wave holds pieces of two rows"
+    # a row's pieces are even, and no longer than the longest piece length
+    for _, it, _ in items:
+        for key in {tuple(r) for r in it[:, [0, 6]].tolist()}:
+            n = [r[5] - r[4] for r in it.tolist() if (r[0], r[6]) == key]
+            assert max(n) - min(n) <= 1 and max(n) <= 12
+
+
 @pytest.mark.parametrize("hq,hkv", [(32, 8), (8, 8), (64, 2)])
 @pytest.mark.parametrize("causal", [1, 0])
 @pytest.mark.parametrize("q_len,kv_len,max_slots", [
