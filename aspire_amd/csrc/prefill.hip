@@ -691,7 +691,8 @@ extern "C" int aspire_prefill_run(const aspire_prefill_args* a, void* stream) {
 extern "C" int aspire_prefill_run_units(const aspire_prefill_args* a, const int32_t* units, int32_t num_units,
                                         const int32_t* merges, int32_t num_merges, int32_t num_slots, float* partials,
                                         int64_t partials_size, void* stream) {
-  if (units == nullptr) return aspire::fail(ASPIRE_ERR_INVALID, "aspire_prefill_run_units: null units");
+  if (units == nullptr && (a == nullptr || (a->num_rows > 0 && a->total_blocks > 0)))  // a batch without queries has none
+    return aspire::fail(ASPIRE_ERR_INVALID, "aspire_prefill_run_units: null units");
   return aspire::prefill_launch(a, units, num_units, merges, num_merges, num_slots, partials, partials_size, stream);
 }
 

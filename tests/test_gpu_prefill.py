@@ -270,3 +270,15 @@ def test_prefill_long_prefix_is_cut_and_matches_whole_blocks(gpu, monkeypatch):
     (a, la), (b, lb) = outs
     attn_close(a, b)
     assert (la - lb).abs().max() < 1e-4
+
+
+def test_prefill_of_a_batch_without_queries(gpu):
+    """Rows that append nothing: the plan lists no work and run() leaves ``out`` as it is."""
+    cache = torch.randn(8, 2, 16, 8, 128, device=gpu).bfloat16()
+    w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(1, device=gpu), "NHD")
+    w.plan(torch.zeros(3, dtype=torch.int32, device=gpu), torch.tensor([0, 3, 8], dtype=torch.int32, device=gpu),
+           torch.arange(8, dtype=torch.int32, device=gpu), torch.tensor([5, 16], dtype=torch.int32, device=gpu), 32, 8, 128, 16,
+           causal=True)
+    out = torch.full((4, 32, 128), 3.0, dtype=torch.bfloat16, device=gpu)
+    w.run(torch.randn(4, 32, 128, device=gpu).bfloat16(), cache, out=out)
+    assert (out == 3.0).all()

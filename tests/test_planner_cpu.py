@@ -438,3 +438,15 @@ def test_prefill_units_cover_every_step_once(hq, hkv, causal, q_len, kv_len, max
             assert count == len(got) and [p[2] for p in got] == list(range(first, first + count))
             used += [p[2] for p in got]
     assert sorted(used) == list(range(slots)) and len(merge_of) == merges
+
+
+def test_prefill_run_units_of_a_batch_without_queries_needs_no_units():
+    lib = _lib.lib()
+    a = _lib.PrefillArgs()
+    a.num_qo_heads, a.num_kv_heads, a.head_dim, a.page_size, a.sm_scale = 32, 8, 128, 16, 1.0
+    a.block_tokens, a.num_rows, a.total_blocks = lib.aspire_prefill_block_tokens(32, 8), 2, 0
+    a.cache_stride_t, a.cache_stride_p = 1024, 32768
+    none = None, 0, None, 0, 0, None, 0, None
+    assert lib.aspire_prefill_run_units(ctypes.byref(a), *none) == 0
+    a.total_blocks = 1
+    assert lib.aspire_prefill_run_units(ctypes.byref(a), *none) == _lib.ASPIRE_ERR_INVALID
