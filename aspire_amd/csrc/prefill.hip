@@ -547,6 +547,17 @@ int piece_count(int32_t steps, int64_t piece) {
   return steps > piece + piece / 4 ? static_cast<int>((steps + piece - 1) / piece) : 1;
 }
 
+// Order units longest first, but only by sixteenths of the longest: units of about one length stay in
+// block order, where neighbours share keys in L2. us, sorted by every step -> by sixteenths: 8 rows of 328
+// to 776 tokens over 29,677 (64/8 heads) 3,637 -> 3,357 (block order 3,346), 6 x 518 over 28,089 1,550 ->
+// 1,425, 8 x 202 over 18,505, cut in four, 543 -> 513. Of 68 batches drawn over 16 to 8,192 tokens and up to
+// 32,768 cached ones the worst lost 2.7% (157 -> 162), the mean gained 1.2%; by fortieths 0.3%.
+void longest_first(std::vector<int32_t>& order, const std::vector<int32_t>& lens) {
+  const int64_t longest = lens.empty() ? 1 : std::max<int32_t>(1, *std::max_element(lens.begin(), lens.end()));
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int32_t x, int32_t y) { return 16 * int64_t(lens[x]) / longest > 16 * int64_t(lens[y]) / longest; });
+}
+
 // A launch's first workgroups go round a head's CUs one each, then a second and a third each, and only
 // later ones wait for a place. So the units (longest first) are dealt out three a CU, each to the CU
 // with the least work that has a place left, and listed by rounds; the rest follow in their order.
@@ -559,28 +570,34 @@ double deal(const std::vector<int32_t>& lens, int cus, std::vector<int32_t>* ord
   std::vector<std::vector<int32_t>> places(cus);
   for (int c = 0; c < cus; ++c) open.push({0.0, c});
   const int n = static_cast<int>(lens.size()), dealt = std::min(n, kPfPerCu * cus);
+  std::vector<int32_t> by(n);
+  for (int i = 0; i < n; ++i) by[i] = i;
+  longest_first(by, lens);
   for (int i = 0; i < dealt; ++i) {
     const Load at = open.top();
     open.pop();
-    places[at.second].push_back(i);
-    if (static_cast<int>(places[at.second].size()) < kPfPerCu) open.push({at.first + lens[i], at.second});
+    places[at.second].push_back(by[i]);
+    if (static_cast<int>(places[at.second].size()) < kPfPerCu) open.push({at.first + lens[by[i]], at.second});
   }
   if (order != nullptr) {
     order->clear();
     for (int round = 0; round < kPfPerCu; ++round)
       for (int c = 0; c < cus; ++c)
         if (round < static_cast<int>(places[c].size())) order->push_back(places[c][round]);
-    for (int i = dealt; i < n; ++i) order->push_back(i);
+    for (int i = dealt; i < n; ++i) order->push_back(by[i]);
   }
   double most = 0;
   std::priority_queue<double, std::vector<double>, std::greater<double>> times;
   for (const auto& p : places) {
-    const double a = p.size() > 0 ? lens[p[0]] : 0, b = p.size() > 1 ? lens[p[1]] : 0, c = p.size() > 2 ? lens[p[2]] : 0;
-    times.push(0.46 * 3 * c + 0.5 * 2 * (b - c) + 0.66 * (a - b));
-    most = std::max(most, 0.46 * 3 * c + 0.5 * 2 * (b - c) + 0.66 * (a - b));
+    double l[kPfPerCu] = {0, 0, 0};
+    for (size_t i = 0; i < p.size(); ++i) l[i] = lens[p[i]];
+    std::sort(l, l + kPfPerCu, std::greater<double>());
+    const double us = 0.46 * 3 * l[2] + 0.5 * 2 * (l[1] - l[2]) + 0.66 * (l[0] - l[1]);
+    times.push(us);
+    most = std::max(most, us);
   }
   for (int i = dealt; i < n; ++i) {
-    const double now = times.top() + 0.46 * lens[i];
+    const double now = times.top() + 0.46 * lens[by[i]];
     times.pop();
     times.push(now);
     most = std::max(most, now);
@@ -596,7 +613,7 @@ double estimate_us(const std::vector<int32_t>& steps, const std::vector<int32_t>
   lens.clear();
   slots = 0;
   double part_bytes = 0;
-  for (size_t i = 0; i < steps.size(); ++i) {
+  for (size_t i = steps.size(); i-- > 0;) {
     const int k = piece_count(steps[i], piece);
     for (int j = 0; j < k; ++j) lens.push_back(static_cast<int32_t>((int64_t(steps[i]) + j) / k) + kPfStart);
     if (k > 1) {
@@ -604,7 +621,6 @@ double estimate_us(const std::vector<int32_t>& steps, const std::vector<int32_t>
       part_bytes += double(k) * rows[i] * num_kv_heads * 1024.0;
     }
   }
-  std::sort(lens.begin(), lens.end(), std::greater<int32_t>());
   return deal(lens, std::max(1, 256 / num_kv_heads), nullptr) + (slots > 0 ? 6.0 + part_bytes / 5e6 : 0.0);
 }
 
@@ -750,14 +766,13 @@ extern "C" int aspire_prefill_plan(const int32_t* q_len, const int32_t* kv_len, 
         units.push_back(Unit{i, at, j + 1 == k ? 0x7fffffff : to, k > 1 ? slots++ : -1, to - at});
       }
     }
-    std::stable_sort(units.begin(), units.end(), [](const Unit& x, const Unit& y) { return x.len > y.len; });
     *num_units = static_cast<int32_t>(units.size());
     *num_merges = static_cast<int32_t>(merges.size() / 4);
     *num_slots = slots;
     if (out != nullptr) {
       ASPIRE_CHECK_ARG(out_size >= int64_t(units.size()) * 4 + int64_t(merges.size()), "out is too small");
       lens.clear();
-      for (const Unit& u : units) lens.push_back(u.len);
+      for (const Unit& u : units) lens.push_back(u.len + kPfStart);
       std::vector<int32_t> order;
       deal(lens, std::max(1, 256 / num_kv_heads), &order);
       for (int32_t i : order) {
