@@ -238,3 +238,29 @@ def test_decode_step_graph_replays_match_eager(gpu, shape):
         assert torch.equal(glogits, e_logits), f"replay {i} logits"
         assert torch.equal(step.selector.selected, e_sel), f"replay {i} selection"
         _ = torch.randn(1000, device=gpu).sum().item()   # eager work between replays
+
+
+@pytest.mark.parametrize("vocab", [1, 7, 8, 8191, 8200, 40960, 40969, 151936])
+def test_argmax_rows_ties_infinities_and_nan(gpu, vocab):
+    """Rows shorter and longer than a round of vectors: the first of equal largest values, rows of -inf (whole,
+    and up to one value), NaN never picked beside a number (past the row's first value, which every thread
+    without a number of its own starts from)."""
+    stride = (vocab + 7) // 8 * 8
+    g = torch.Generator().manual_seed(vocab)
+    x = torch.randn(8, stride, generator=g).bfloat16()
+    x[1] = -float("inf")
+    x[2] = -float("inf")
+    x[2, vocab - 1] = -3e38
+    x[3] = 2.0
+    x[4, 1 : vocab // 2] = float("nan")
+    x[5, torch.randint(0, vocab, (5,), generator=g)] = 100.0
+    x[6] = -1.0
+    x[6, vocab // 3:] = -float("inf")
+    x[7, : vocab // 2] = -0.0
+    x[7, vocab // 2:] = 0.0
+    ids = torch.empty(8, dtype=torch.int64, device=gpu)
+    argmax_rows(x.to(gpu)[:, :vocab], ids)
+    v = x[:, :vocab].float()
+    v = torch.where(v.isnan(), -torch.inf, v)
+    first = (v == v.max(dim=1, keepdim=True).values).to(torch.int8).argmax(dim=1)
+    assert ids.cpu().tolist() == first.tolist()
