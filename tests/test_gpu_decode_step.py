@@ -247,7 +247,7 @@ def test_argmax_rows_ties_infinities_and_nan(gpu, vocab):
     without a number of its own starts from)."""
     stride = (vocab + 7) // 8 * 8
     g = torch.Generator().manual_seed(vocab)
-    x = torch.randn(8, stride, generator=g).bfloat16()
+    x = torch.randn(9, stride, generator=g).bfloat16()
     x[1] = -float("inf")
     x[2] = -float("inf")
     x[2, vocab - 1] = -3e38
@@ -258,7 +258,10 @@ def test_argmax_rows_ties_infinities_and_nan(gpu, vocab):
     x[6, vocab // 3:] = -float("inf")
     x[7, : vocab // 2] = -0.0
     x[7, vocab // 2:] = 0.0
-    ids = torch.empty(8, dtype=torch.int64, device=gpu)
+    x[8] = -float("inf")                     # a masked row: vectors of NaN, of -inf, one with a subnormal
+    x[8, 1 : vocab // 3] = float("nan")
+    x[8, vocab // 2] = 1e-40
+    ids = torch.empty(9, dtype=torch.int64, device=gpu)
     argmax_rows(x.to(gpu)[:, :vocab], ids)
     v = x[:, :vocab].float()
     v = torch.where(v.isnan(), -torch.inf, v)
