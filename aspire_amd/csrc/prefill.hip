@@ -440,7 +440,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
         *reinterpret_cast<float4*>(dst + 32 * (c >> 1) + 8 * grp + 4 * (c & 1)) =
             make_float4(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
       }
-      if (grp == 0) p.part_lse[slot] = lse_v;
+      if (grp == 0) p.part_lse[slot] = lt == 0.f || lt > 0.f ? lse_v : lt;  // a sum of NaN stays one in the merge
       continue;
     }
     uint16_t* dst = p.out + int64_t(token) * p.o_st + int64_t(head) * p.o_sh;
@@ -501,7 +501,14 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p, con
     float top = mx;
 #pragma unroll
     for (int i = 0; i < kRound; ++i) top = fmaxf(top, l[i]);
-    if (top == kNegInfP) continue;
+    if (top == kNegInfP) {  // no visible key so far: zeros, or the NaN of a query that has one
+#pragma unroll
+      for (int i = 0; i < kRound; ++i) {
+        o[0] += x[i].x, o[1] += x[i].y, o[2] += x[i].z, o[3] += x[i].w;
+        o[4] += y[i].x, o[5] += y[i].y, o[6] += y[i].z, o[7] += y[i].w;
+      }
+      continue;
+    }
     const float keep = __builtin_amdgcn_exp2f(mx - top);
     sum *= keep;
 #pragma unroll

@@ -282,3 +282,37 @@ def test_prefill_of_a_batch_without_queries(gpu):
     out = torch.full((4, 32, 128), 3.0, dtype=torch.bfloat16, device=gpu)
     w.run(torch.randn(4, 32, 128, device=gpu).bfloat16(), cache, out=out)
     assert (out == 3.0).all()
+
+
+def test_prefill_pieces_carry_nan_and_infinity(gpu, monkeypatch):
+    """NaN and infinite queries, keys and values in rows whose blocks are cut: NaN outputs and LSEs where the same
+    blocks taken whole have them (a query of NaN sees no finite key in any piece), the same numbers elsewhere."""
+    say("prefill pieces, nan")
+    step = build_step(hq=32, hkv=8, ctx_len=[700, 300], q_len=[40, 9], is_draft=[0, 0], draft_budget=0, seed=42, device=gpu)
+    args = (step.qo_indptr[:-1], step.kv_indptr[:-1], step.kv_indices, step.last_page_len[:-1], 32, 8, 128, PAGE)
+    q, cache = step.q.clone(), step.cache.clone()
+    table = step.block_table.cpu().numpy()
+    q[3, 5, 7] = float("nan")
+    q[11] = float("nan")
+    q[17, 2] = 3e38                                              # scores of +-inf
+    cache[int(table[0, 20]), 0, 3, 1, 9] = float("nan")          # a key and a value in the middle of row 0
+    cache[int(table[0, 30]), 1, 4, 2, 60] = float("nan")
+    cache[int(table[1, 2]), 1, 1, 3, 100] = float("inf")
+    outs = []
+    for cut in (False, True):
+        def plan_units(ql, kl, bt, *rest, cut=cut):
+            return _pieces(step, bt, 3 if cut else 10**6, True)
+
+        monkeypatch.setattr(BatchPrefillWithPagedKVCacheWrapper, "_plan_units", staticmethod(plan_units))
+        w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(1, device=gpu), "NHD")
+        w.plan(*args, causal=True)
+        assert (w._pf["slots"] > 0) == cut
+        outs.append(w.run(q, cache, return_lse=True))
+    (a, la), (b, lb) = ((x[: step.total_tokens].float().cpu() for x in o) for o in outs)
+    assert a[11].isnan().all() and a.isnan().any(dim=-1)[40:, 12:16].sum() == 0
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+    ok = a.isfinite()
+    assert (a[ok] - b[ok]).abs().max() < 2e-2
+    assert torch.equal(la.isnan(), lb.isnan()) and torch.equal(la.isinf(), lb.isinf())
+    ok = la.isfinite()
+    assert (la[ok] - lb[ok]).abs().max() < 2e-3
