@@ -168,12 +168,18 @@ class BatchPrefillWithPagedKVCacheWrapper(HolisticAttentionWrapper):
         a.num_qo_heads, a.num_kv_heads, a.head_dim, a.page_size = self._num_qo_heads, self._num_kv_heads, 128, 16
         a.sm_scale = float(self._sm_scale if self._sm_scale is not None else 1.0 / math.sqrt(128))
         a.causal = 1 if self._causal else 0
-        # a buffer of this call's own (from torch's pool): runs on several streams do not share it
+        # a buffer of this call's own (from torch's pool): runs on several streams do not share it. Where the
+        # card has no room for it the blocks are run whole, which takes longer and needs none.
+        L = _lib.lib()
         size = pf["slots"] * self._num_kv_heads * (pf["block_tokens"] * self._num_qo_heads // self._num_kv_heads) * 129
-        partials = torch.empty(size, dtype=torch.float32, device=q.device) if size else None
-        rc = _lib.lib().aspire_prefill_run_units(
-            ctypes.byref(a), _lib.ptr(pf["units"]), pf["units"].shape[0], _lib.ptr(pf["merges"]),
-            pf["merges"].shape[0], pf["slots"], _lib.ptr(partials), size, _lib.stream_of(q))
+        try:
+            partials = torch.empty(size, dtype=torch.float32, device=q.device) if size else None
+        except torch.OutOfMemoryError:
+            rc = L.aspire_prefill_run(ctypes.byref(a), _lib.stream_of(q))
+        else:
+            rc = L.aspire_prefill_run_units(
+                ctypes.byref(a), _lib.ptr(pf["units"]), pf["units"].shape[0], _lib.ptr(pf["merges"]),
+                pf["merges"].shape[0], pf["slots"], _lib.ptr(partials), size, _lib.stream_of(q))
         _lib.check(rc, "BatchPrefillWithPagedKVCacheWrapper.run")
         return (out, lse) if return_lse else out
 

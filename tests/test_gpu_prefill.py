@@ -316,3 +316,33 @@ def test_prefill_pieces_carry_nan_and_infinity(gpu, monkeypatch):
     assert torch.equal(la.isnan(), lb.isnan()) and torch.equal(la.isinf(), lb.isinf())
     ok = la.isfinite()
     assert (la[ok] - lb[ok]).abs().max() < 2e-3
+
+
+def test_prefill_without_room_for_partials_runs_whole_blocks(gpu, monkeypatch):
+    """A cut batch on a card that cannot hold the partial rows: the blocks run whole (aspire_prefill_run), within
+    bf16 rounding of the cut run and against the oracle."""
+    say("prefill, no room for partials")
+    ctx, q_len = [3001, 40, 517], [65, 40, 3]
+    step = build_step(hq=32, hkv=8, ctx_len=ctx, q_len=q_len, is_draft=[0] * 3, draft_budget=0, seed=43, device=gpu)
+    w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(1, device=gpu), "NHD")
+    w.plan(step.qo_indptr[:-1], step.kv_indptr[:-1], step.kv_indices, step.last_page_len[:-1], 32, 8, 128, PAGE, causal=True)
+    size = w._pf["slots"] * 128 * 8 * 129
+    assert size > 0
+    cut, cut_lse = w.run(step.q, step.cache, return_lse=True)
+    empty = torch.empty
+
+    def full(*shape, **kw):
+        if shape == (size,):
+            raise torch.OutOfMemoryError("no room")
+        return empty(*shape, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    out, lse = w.run(step.q, step.cache, return_lse=True)
+    monkeypatch.undo()
+    T = step.total_tokens
+    attn_close(out[:T], cut[:T])
+    assert (lse[:T] - cut_lse[:T]).abs().max() < 1e-4
+    ref_out, ref_lse = paged_attention(step.q.cpu(), step.cache.cpu(), step.qo_indptr_host, step.kv_indptr_host,
+                                       step.kv_indices.cpu(), step.kv_len_host, num_kv_heads=8, causal=True)
+    attn_close(out[:T], ref_out[:T])
+    assert (lse[:T].cpu() - ref_lse[:T]).abs().max() < 2e-3
