@@ -227,8 +227,7 @@ def _declare(lib):
         "aspire_verify_topk_speculation": [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp],
         "aspire_prefill_block_tokens": [i32, i32],
         "aspire_prefill_run": [ctypes.POINTER(PrefillArgs), vp],
-        "aspire_prefill_plan": [vp, vp, i32, i32, i32, i32, i64, vp, i64, ctypes.POINTER(i32), ctypes.POINTER(i32),
-                                ctypes.POINTER(i32)],
+        "aspire_prefill_plan": [vp, vp, i32, i32, i32, i32, i64, vp, i64, vp, vp, vp],
         "aspire_prefill_run_units": [ctypes.POINTER(PrefillArgs), vp, i32, vp, i32, i32, vp, i64, vp],
         "aspire_linear": [vp, i64, vp, i64, vp, i64, i32, i32, i32, i32, vp],
         "aspire_linear_splits": [i32, i32, i32],

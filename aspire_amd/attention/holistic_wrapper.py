@@ -29,6 +29,7 @@ import ctypes
 import math
 from typing import List, Optional, Tuple, Union
 
+import numpy as np
 import torch
 
 from aspire_amd import _lib
@@ -237,9 +238,11 @@ class HolisticAttentionWrapper:
             kvp = kv_indptr_host.to(torch.int32).contiguous()
             if qo.shape[0] < batch + 1 or kvp.shape[0] < n_seg + 1:
                 raise ValueError("plan arrays are shorter than the batch they describe")
-            if n_seg and int(kvp[: n_seg + 1].max()) > paged_kv_indices.numel():
+            if n_seg and kvp.numpy()[: n_seg + 1].max() > paged_kv_indices.numel():
                 raise ValueError("paged_kv_indices is shorter than kv_indptr describes")
-        if int(qo[: batch + 1].min()) < 0:
+        # (numpy on the host arrays: a torch operation costs a few us of the plan, each)
+        qo_np, kvl_np = qo.numpy()[: batch + 1], kvl.numpy()
+        if qo_np.min() < 0:
             raise ValueError("qo_indptr must be non-negative")
         slot = self._pinned_slot
         event = self._pinned_ring_events[slot]
@@ -274,16 +277,15 @@ class HolisticAttentionWrapper:
         self._plan_class_mask = sum(1 << c for c in range(3) if info.num_items[c] > 0)
         self._plan_merge = 1 if info.num_merge > 0 else 0
         self._plan_nt = 1 if info.total_pages <= SHORT_PLAN_PAGES_PER_WAVE * self._layout.num_waves else 0
-        self._plan_tokens = int(qo[: batch + 1].max()) if batch else 0
+        self._plan_tokens = int(qo_np.max()) if batch else 0
         # rows that can write dump entries / page scores: queries and at least one page
         if per_head_lists:
-            has_kv = (kvl[: batch * num_kv_heads].view(batch, num_kv_heads) > 0).any(dim=1) if batch else kvl[:0]
+            has_kv = (kvl_np[: batch * num_kv_heads].reshape(batch, num_kv_heads) > 0).any(axis=1)
         else:
-            has_kv = kvl[:batch] > 0
-        writes = ((qo[1 : batch + 1] - qo[:batch]) > 0) & has_kv
-        nz = torch.nonzero(writes)
-        self._plan_batch = int(nz.max()) + 1 if nz.numel() else 0
-        self._plan_max_kv = int(kvl.max()) if n_seg else 0
+            has_kv = kvl_np[:batch] > 0
+        nz = np.flatnonzero((qo_np[1:] > qo_np[:-1]) & has_kv)
+        self._plan_batch = int(nz[-1]) + 1 if nz.size else 0
+        self._plan_max_kv = int(kvl_np.max()) if n_seg else 0
         self._plan_max_pages = (self._plan_max_kv + page_size - 1) // page_size
         self._kv_indices = paged_kv_indices
         self._page_size = page_size

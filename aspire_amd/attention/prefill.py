@@ -28,6 +28,7 @@ import ctypes
 import math
 from typing import Optional, Union
 
+import numpy as np
 import torch
 
 from aspire_amd import _lib
@@ -84,17 +85,17 @@ class BatchPrefillWithPagedKVCacheWrapper(HolisticAttentionWrapper):
         # rows: the entries of kv_last_page_len (FlashInfer's batch), with their query blocks; the
         # plan above has read the lengths back
         n = paged_kv_last_page_len.shape[0]
-        qo_host, kv_len = (t.to(torch.int64) for t in self._plan_host_lens)
-        q_len = (qo_host[1 : n + 1] - qo_host[:n]).clamp(min=0)
-        blocks = torch.zeros(n + 1, dtype=torch.int64)
-        blocks[1:] = torch.cumsum((q_len + bt - 1) // bt, 0)
+        qo_host, kv_len = (t.numpy() for t in self._plan_host_lens)  # int32
+        q_len = np.maximum(qo_host[1 : n + 1] - qo_host[:n], 0)
+        blocks = np.zeros(n + 1, dtype=np.int32)
+        np.cumsum((q_len + (bt - 1)) // bt, out=blocks[1:])
+        total = int(blocks[n])
+        units, merges, slots = self._plan_units(q_len, kv_len[:n], bt, num_qo_heads, num_kv_heads, causal, total)
+        nu, at = units.numel(), units.numel() + merges.numel()
         dev = paged_kv_indices.device
-        total = int(blocks[-1])
-        units, merges, slots = self._plan_units(q_len, kv_len[:n], bt, num_qo_heads, num_kv_heads, causal)
-        tables = torch.cat([units.view(-1), merges.view(-1), blocks.to(torch.int32)]).to(dev)  # one upload
-        at = units.numel() + merges.numel()
+        tables = torch.cat([units.view(-1), merges.view(-1), torch.from_numpy(blocks)]).to(dev)  # one upload
         self._pf = {
-            "units": tables[: units.numel()].view(-1, 4), "merges": tables[units.numel() : at].view(-1, 4), "slots": slots,
+            "units": tables[:nu].view(-1, 4), "merges": tables[nu:at].view(-1, 4), "slots": slots,
             "qo": qo_indptr[: n + 1].to(dev, torch.int32).contiguous(),
             "kvp": paged_kv_indptr[: n + 1].to(dev, torch.int32).contiguous(),
             "lpl": paged_kv_last_page_len[:n].to(dev, torch.int32).contiguous(),
@@ -105,22 +106,21 @@ class BatchPrefillWithPagedKVCacheWrapper(HolisticAttentionWrapper):
         }
 
     @staticmethod
-    def _plan_units(q_len, kv_len, block_tokens, num_qo_heads, num_kv_heads, causal):
-        """``(units [U, 4], merges [M, 4], partial slots)`` for the prefill kernel: the query blocks dealt out
-        over the CUs, the long ones cut along their keys where whole blocks would leave the chip idle or uneven."""
-        n = q_len.shape[0]
-        ql, kl = q_len.to(torch.int32).contiguous(), kv_len.to(torch.int32).contiguous()
+    def _plan_units(q_len, kv_len, block_tokens, num_qo_heads, num_kv_heads, causal, blocks):
+        """``(units [U, 4], merges [M, 4], partial slots)`` for the prefill kernel, from int32 numpy lengths and the
+        number of query blocks: the blocks dealt out over the CUs, the long ones cut along their keys where whole
+        blocks would leave the chip idle or uneven."""
         block_rows = block_tokens * num_qo_heads // num_kv_heads
         most = PARTIAL_BYTES // (num_kv_heads * block_rows * 129 * 4)
-        counts = [ctypes.c_int32() for _ in range(3)]
-        # room for the largest tables: a unit and a merge a block, and every slot a unit
-        blocks = int(((q_len + block_tokens - 1) // block_tokens).sum())
-        table = torch.empty((2 * blocks + most, 4), dtype=torch.int32)
-        rc = _lib.lib().aspire_prefill_plan(_lib.ptr(ql), _lib.ptr(kl), n, num_qo_heads, num_kv_heads, 1 if causal else 0,
-                                            most, _lib.ptr(table), table.numel(), *(ctypes.byref(c) for c in counts))
+        ql, kl = torch.from_numpy(q_len), torch.from_numpy(np.ascontiguousarray(kv_len))
+        # three counts, then room for the largest tables: a unit and a merge a block, and every slot a unit
+        table = torch.empty((1 + 2 * blocks + most, 4), dtype=torch.int32)
+        at = table.data_ptr()
+        rc = _lib.lib().aspire_prefill_plan(ql.data_ptr(), kl.data_ptr(), ql.numel(), num_qo_heads, num_kv_heads,
+                                            1 if causal else 0, most, at + 16, table.numel() - 4, at, at + 4, at + 8)
         _lib.check(rc, "plan")
-        n_units, n_merges, slots = (c.value for c in counts)
-        return table[:n_units], table[n_units : n_units + n_merges], slots
+        n_units, n_merges, slots = table[0, :3].tolist()
+        return table[1 : 1 + n_units], table[1 + n_units : 1 + n_units + n_merges], slots
 
     def run(self, q: torch.Tensor, paged_kv_cache, *args, out: Optional[torch.Tensor] = None,
             lse: Optional[torch.Tensor] = None, return_lse: bool = False, **kwargs):

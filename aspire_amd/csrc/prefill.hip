@@ -31,7 +31,7 @@
 // Waves whose tokens end before a step skip its compute but keep staging.
 #include <algorithm>
 #include <functional>
-#include <queue>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -554,88 +554,147 @@ int piece_count(int32_t steps, int64_t piece) {
   return steps > piece + piece / 4 ? static_cast<int>((steps + piece - 1) / piece) : 1;
 }
 
+// The buffers of one plan, reused for every piece length that is tried.
+struct Dealing {
+  std::vector<int32_t> lens, by, order;
+  std::vector<uint8_t> bucket;
+  std::vector<int32_t> places;            // [cus][kPfPerCu] units, `held` of them
+  std::vector<int8_t> held;
+  std::vector<std::pair<int64_t, int>> open;  // heaps, least first
+  std::vector<double> times;
+};
+
+// The least element of a heap was raised: put it in its place.
+template <typename T>
+void sift_down(std::vector<T>& heap) {
+  const size_t n = heap.size();
+  const T v = heap[0];
+  size_t i = 0;
+  for (size_t c = 1; c < n; c = 2 * i + 1) {
+    if (c + 1 < n && heap[c + 1] < heap[c]) ++c;
+    if (!(heap[c] < v)) break;
+    heap[i] = heap[c];
+    i = c;
+  }
+  heap[i] = v;
+}
+
 // Order units longest first, but only by sixteenths of the longest: units of about one length stay in
 // block order, where neighbours share keys in L2. us, sorted by every step -> by sixteenths: 8 rows of 328
 // to 776 tokens over 29,677 (64/8 heads) 3,637 -> 3,357 (block order 3,346), 6 x 518 over 28,089 1,550 ->
 // 1,425, 8 x 202 over 18,505, cut in four, 543 -> 513. Of 68 batches drawn over 16 to 8,192 tokens and up to
 // 32,768 cached ones the worst lost 2.7% (157 -> 162), the mean gained 1.2%; by fortieths 0.3%.
-std::vector<int32_t> longest_first(const std::vector<int32_t>& lens) {
+void longest_first(Dealing& d) {
+  const std::vector<int32_t>& lens = d.lens;
   const int64_t longest = lens.empty() ? 1 : std::max<int32_t>(1, *std::max_element(lens.begin(), lens.end()));
   const double scale = 16.0 / static_cast<double>(longest);
   int32_t at[18] = {0};  // a counting sort: this runs for every piece length that is tried
-  std::vector<uint8_t> bucket(lens.size());
+  d.bucket.resize(lens.size());
   for (size_t i = 0; i < lens.size(); ++i) {
-    bucket[i] = static_cast<uint8_t>(16 - std::min(16, static_cast<int>(scale * lens[i])));
-    ++at[bucket[i] + 1];
+    d.bucket[i] = static_cast<uint8_t>(16 - std::min(16, static_cast<int>(scale * lens[i])));
+    ++at[d.bucket[i] + 1];
   }
   for (int k = 1; k < 18; ++k) at[k] += at[k - 1];
-  std::vector<int32_t> order(lens.size());
-  for (size_t i = 0; i < lens.size(); ++i) order[at[bucket[i]]++] = static_cast<int32_t>(i);
-  return order;
+  d.by.resize(lens.size());
+  for (size_t i = 0; i < lens.size(); ++i) d.by[at[d.bucket[i]]++] = static_cast<int32_t>(i);
 }
 
 // A launch's first workgroups go round a head's CUs one each, then a second and a third each, and only
 // later ones wait for a place. So the units (longest first) are dealt out three a CU, each to the CU
 // with the least work that has a place left, and listed by rounds; the rest follow in their order.
-// Returns the estimated us of the slowest CU: 0.66 us a step for a workgroup by itself, 0.5 for
+void deal(Dealing& d, int cus) {
+  const std::vector<int32_t>& lens = d.lens;
+  const int n = static_cast<int>(lens.size()), dealt = std::min(n, kPfPerCu * cus);
+  longest_first(d);
+  d.places.resize(size_t(cus) * kPfPerCu);
+  d.held.assign(cus, 0);
+  d.open.clear();
+  for (int c = 0; c < cus; ++c) {  // the first round goes to every CU in turn
+    const int32_t unit = c < dealt ? d.by[c] : 0;
+    d.places[c * kPfPerCu] = unit;
+    d.held[c] = c < dealt;
+    d.open.emplace_back(c < dealt ? lens[unit] : 0, c);
+  }
+  if (dealt > cus) std::make_heap(d.open.begin(), d.open.end(), std::greater<std::pair<int64_t, int>>());
+  for (int i = cus; i < dealt; ++i) {
+    const int c = d.open[0].second;
+    d.places[c * kPfPerCu + d.held[c]] = d.by[i];
+    if (++d.held[c] < kPfPerCu) {
+      d.open[0].first += lens[d.by[i]];
+    } else {
+      d.open[0] = d.open.back();
+      d.open.pop_back();
+    }
+    if (!d.open.empty()) sift_down(d.open);
+  }
+}
+
+void list_units(Dealing& d, int cus) {
+  const size_t dealt = std::min(d.lens.size(), size_t(cus) * kPfPerCu);
+  d.order.clear();
+  for (int round = 0; round < kPfPerCu; ++round)
+    for (int c = 0; c < cus; ++c)
+      if (round < d.held[c]) d.order.push_back(d.places[c * kPfPerCu + round]);
+  d.order.insert(d.order.end(), d.by.begin() + dealt, d.by.end());
+}
+
+// The estimated us of the slowest CU of dealt units: 0.66 us a step for a workgroup by itself, 0.5 for
 // each of two workgroups' steps and 0.46 for each of three's (8,192 tokens: 263,000 steps of all heads
 // in 470 us).
-double deal(const std::vector<int32_t>& lens, int cus, std::vector<int32_t>* order) {
-  typedef std::pair<double, int> Load;
-  std::priority_queue<Load, std::vector<Load>, std::greater<Load>> open;
-  std::vector<std::vector<int32_t>> places(cus);
-  for (int c = 0; c < cus; ++c) open.push({0.0, c});
+constexpr double kUsAlone = 0.66, kUsTwo = 0.5, kUsThree = 0.46;
+
+double slowest_us(Dealing& d, int cus) {
+  const std::vector<int32_t>& lens = d.lens;
   const int n = static_cast<int>(lens.size()), dealt = std::min(n, kPfPerCu * cus);
-  const std::vector<int32_t> by = longest_first(lens);
-  for (int i = 0; i < dealt; ++i) {
-    const Load at = open.top();
-    open.pop();
-    places[at.second].push_back(by[i]);
-    if (static_cast<int>(places[at.second].size()) < kPfPerCu) open.push({at.first + lens[by[i]], at.second});
-  }
-  if (order != nullptr) {
-    order->clear();
-    for (int round = 0; round < kPfPerCu; ++round)
-      for (int c = 0; c < cus; ++c)
-        if (round < static_cast<int>(places[c].size())) order->push_back(places[c][round]);
-    for (int i = dealt; i < n; ++i) order->push_back(by[i]);
-  }
   double most = 0;
-  std::priority_queue<double, std::vector<double>, std::greater<double>> times;
-  for (const auto& p : places) {
+  d.times.clear();
+  for (int c = 0; c < cus; ++c) {
     double l[kPfPerCu] = {0, 0, 0};
-    for (size_t i = 0; i < p.size(); ++i) l[i] = lens[p[i]];
+    for (int i = 0; i < d.held[c]; ++i) l[i] = lens[d.places[c * kPfPerCu + i]];
     std::sort(l, l + kPfPerCu, std::greater<double>());
-    const double us = 0.46 * 3 * l[2] + 0.5 * 2 * (l[1] - l[2]) + 0.66 * (l[0] - l[1]);
-    times.push(us);
+    const double us = kUsThree * 3 * l[2] + kUsTwo * 2 * (l[1] - l[2]) + kUsAlone * (l[0] - l[1]);
+    d.times.push_back(us);
     most = std::max(most, us);
   }
+  if (dealt < n) std::make_heap(d.times.begin(), d.times.end(), std::greater<double>());
   for (int i = dealt; i < n; ++i) {
-    const double now = times.top() + 0.46 * lens[by[i]];
-    times.pop();
-    times.push(now);
-    most = std::max(most, now);
+    d.times[0] += kUsThree * lens[d.by[i]];
+    most = std::max(most, d.times[0]);
+    sift_down(d.times);
   }
   return most;
 }
 
 // Estimated us of a launch with the blocks cut at `piece` steps: every piece's rows are written and
-// read once in fp32 (about 5 TB/s) and merged by a launch of its own. The heads' workgroups go round
-// the XCDs, so a head has about 256 / num_kv_heads CUs.
+// read once in fp32 (about 5 TB/s) and merged by a launch of its own. At least `best` where the CUs' mean
+// (no step takes less than kUsThree) says that it cannot be less: dealing the units out is most of a
+// plan's time. With that, with whole blocks dealt once where no piece length cuts any, and with heaps kept from
+// one estimate to the next, aspire_prefill_plan takes (us of one host core, before -> now): 8,192 tokens 31 ->
+// 10, 5 rows of 17 to 700 tokens over 300 to 8,000 60 -> 17, 8 x 1,000 over 2,000 (64/2 heads) 208 -> 39.
 double estimate_us(const std::vector<int32_t>& steps, const std::vector<int32_t>& rows, int64_t piece, int num_kv_heads,
-                   std::vector<int32_t>& lens, int64_t& slots) {
-  lens.clear();
+                   int cus, double best, Dealing& d, int64_t& slots) {
   slots = 0;
   double part_bytes = 0;
-  for (size_t i = steps.size(); i-- > 0;) {
+  int64_t units = 0, total = 0;
+  for (size_t i = 0; i < steps.size(); ++i) {
     const int k = piece_count(steps[i], piece);
-    for (int j = 0; j < k; ++j) lens.push_back(static_cast<int32_t>((int64_t(steps[i]) + j) / k) + kPfStart);
+    units += k;
+    total += steps[i];
     if (k > 1) {
       slots += k;
       part_bytes += double(k) * rows[i] * num_kv_heads * 1024.0;
     }
   }
-  return deal(lens, std::max(1, 256 / num_kv_heads), nullptr) + (slots > 0 ? 6.0 + part_bytes / 5e6 : 0.0);
+  const double merge = 6.0 + part_bytes / 5e6;
+  const double least = kUsThree * double(total + kPfStart * units) / cus * (1 - 1e-9) + merge;
+  if (least >= best) return least;
+  d.lens.clear();
+  for (size_t i = steps.size(); i-- > 0;) {
+    const int k = piece_count(steps[i], piece);
+    for (int j = 0; j < k; ++j) d.lens.push_back(static_cast<int32_t>((int64_t(steps[i]) + j) / k) + kPfStart);
+  }
+  deal(d, cus);
+  return slowest_us(d, cus) + merge;
 }
 
 int prefill_launch(const aspire_prefill_args* a, const int32_t* units, int32_t num_units, const int32_t* merges,
@@ -751,18 +810,25 @@ extern "C" int aspire_prefill_plan(const int32_t* q_len, const int32_t* kv_len, 
     // slots (16 steps at least), whichever the estimate likes best. Whole -> cut, us: 64 tokens over
     // 16,000 332 -> 38, 5 rows of 17 to 700 tokens over 300 to 8,192 196 -> 158, 300 over 8,000 171 -> 60.
     int64_t piece = int64_t(1) << 40, slots_of;
+    const int cus = std::max(1, 256 / num_kv_heads);  // the heads' workgroups go round the XCDs
     const int32_t longest = n > 0 ? *std::max_element(steps.begin(), steps.end()) : 0;
-    int64_t last = 0;
-    std::vector<int32_t> lens;
-    double best = estimate_us(steps, rows_of, piece, num_kv_heads, lens, slots_of);
-    for (double f = 2.5; f >= 0.5; f -= 0.25) {
-      const int64_t cut = std::max<int64_t>(16, int64_t(f * double(total) * num_kv_heads / 768));
-      if (piece_count(longest, cut) == 1 || (f < 2.5 && cut == last)) continue;  // whole blocks, or the same pieces again
-      last = cut;
-      const double us = estimate_us(steps, rows_of, cut, num_kv_heads, lens, slots_of);
-      if (us < best && slots_of <= max_slots) {
-        best = us;
-        piece = cut;
+    const auto cut_at = [&](double f) { return std::max<int64_t>(16, int64_t(f * double(total) * num_kv_heads / 768)); };
+    Dealing d;
+    for (int i = n - 1; i >= 0; --i) d.lens.push_back(steps[i] + kPfStart);
+    deal(d, cus);
+    list_units(d, cus);
+    if (piece_count(longest, cut_at(0.5)) > 1) {
+      double best = slowest_us(d, cus);
+      int64_t last = 0;
+      for (double f = 2.5; f >= 0.5; f -= 0.25) {
+        const int64_t cut = cut_at(f);
+        if (piece_count(longest, cut) == 1 || cut == last) continue;  // whole blocks, or the same pieces again
+        last = cut;
+        const double us = estimate_us(steps, rows_of, cut, num_kv_heads, cus, best, d, slots_of);
+        if (us < best && slots_of <= max_slots) {
+          best = us;
+          piece = cut;
+        }
       }
     }
     struct Unit {
@@ -785,11 +851,13 @@ extern "C" int aspire_prefill_plan(const int32_t* q_len, const int32_t* kv_len, 
     *num_slots = slots;
     if (out != nullptr) {
       ASPIRE_CHECK_ARG(out_size >= int64_t(units.size()) * 4 + int64_t(merges.size()), "out is too small");
-      lens.clear();
-      for (const Unit& u : units) lens.push_back(u.len + kPfStart);
-      std::vector<int32_t> order;
-      deal(lens, std::max(1, 256 / num_kv_heads), &order);
-      for (int32_t i : order) {
+      if (slots > 0) {  // whole blocks are listed already
+        d.lens.clear();
+        for (const Unit& u : units) d.lens.push_back(u.len + kPfStart);
+        deal(d, cus);
+        list_units(d, cus);
+      }
+      for (int32_t i : d.order) {
         const Unit& u = units[i];
         *out++ = u.blk;
         *out++ = u.begin;

@@ -450,3 +450,21 @@ def test_prefill_run_units_of_a_batch_without_queries_needs_no_units():
     assert lib.aspire_prefill_run_units(ctypes.byref(a), *none) == 0
     a.total_blocks = 1
     assert lib.aspire_prefill_run_units(ctypes.byref(a), *none) == _lib.ASPIRE_ERR_INVALID
+
+
+@pytest.mark.parametrize("hq,hkv,t,p,want", [
+    (32, 8, [8192], [0], (256, 0, 0)), (32, 8, [2048], [0], (64, 0, 0)), (32, 8, [512], [4096], (64, 16, 64)),
+    (32, 8, [64], [16000], (64, 2, 64)), (32, 8, [17, 400, 700, 90, 333], [300, 8000, 4000, 2000, 900], (98, 35, 83)),
+    (64, 2, [1000] * 8, [2000] * 8, (2000, 0, 0)), (8, 8, [300] * 32, [3000] * 32, (96, 0, 0)),
+    (32, 8, [1] * 64, [9000] * 64, (128, 64, 128))])
+def test_prefill_plan_skips_no_piece_length_that_is_better(hq, hkv, t, p, want):
+    """Units, merges and slots that the estimate of every piece length chooses: lengths that are passed over because
+    they cannot be better, and whole blocks that are not estimated, change none of it."""
+    import torch
+
+    ql = torch.tensor(t, dtype=torch.int32)
+    kl = ql + torch.tensor(p, dtype=torch.int32)
+    n = torch.zeros(3, dtype=torch.int32)
+    at = [n.data_ptr() + 4 * i for i in range(3)]
+    assert _lib.lib().aspire_prefill_plan(_lib.ptr(ql), _lib.ptr(kl), len(t), hq, hkv, 1, 508, None, 0, *at) == 0
+    assert tuple(n.tolist()) == want
