@@ -85,7 +85,7 @@ def test_supported_shapes(gpu):
         linear_partials(x, w, torch.empty(8, device=gpu))
 
 
-@pytest.mark.parametrize("rows,dim,splits", [(1, 8, 1), (37, 4096, 4), (5, 512, 3), (3, 8192, 8)])
+@pytest.mark.parametrize("rows,dim,splits", [(1, 8, 1), (37, 4096, 4), (5, 512, 3), (3, 8192, 8), (2, 1024, 9), (3, 520, 17)])
 def test_add_rms_norm_partials(gpu, rows, dim, splits):
     """Equal, bit for bit, to add_rms_norm with the slabs' sum rounded to bf16."""
     say("add_rms_norm partials", rows, dim, splits)
