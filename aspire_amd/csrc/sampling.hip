@@ -2,11 +2,10 @@
 //
 // * topk_candidates_kernel: the top_k logits of a row and their ids, descending, ties to the
 //   lower id. One 1024-thread workgroup per row, 16-byte loads; rows of up to 155,648 logits
-//   are read once and kept in registers. For up to 128 candidates of such rows, the k-th largest
-//   of 256 group maxima bounds the k-th logit from below, and the few logits at or above that
-//   bound are ranked by counting (see topk_by_maxima). Where that does not settle it, and for
-//   every other row, radix select on 16-bit order-preserving keys
-//   of the bf16 logits: the high byte of the k-th key (for register-held rows from counts at
+//   are read once and kept in registers. For up to 128 candidates of such rows of 8,192 logits or
+//   more, the k-th largest of 256 group maxima bounds the k-th logit from below, and the few logits at
+//   or above that bound are ranked by counting (topk_few_kernel). For every other row, radix select on
+//   16-bit order-preserving keys of the bf16 logits: the high byte of the k-th key (for register-held rows from counts at
 //   the top bins below the row's maximum, else from a histogram), then a histogram of the low
 //   byte among that bin, give the k-th key exactly (each boundary from suffix sums in one
 //   wave); every key at or above it is collected (for register-held rows from the keys of the
@@ -214,83 +213,220 @@ constexpr int kTkCandCap = 2048;    // candidates sorted in LDS
 constexpr int kTkResident = 19;     // 16-byte vectors per thread held in registers (rows up to 155,648 logits)
 constexpr int kTkMaxVocab = 16000000;  // keeps every 16-bit sub-histogram counter below 65,536
 constexpr int kTkGroups = kTkThreads / 4;  // groups of 4 threads whose maxima bound the k-th logit
-constexpr int kTkMaximaK = 128;            // candidates up to which the maxima are tried
+constexpr int kTkMaximaK = 128;            // candidates up to which topk_few_kernel takes a row
 constexpr int kTkRanked = 512;             // logits at or above the bound that are ranked by counting
+static_assert(kTkRanked - kTkMaximaK - 7 >= kTkMaximaK, "ties past kTkRanked: whole vectors hold enough of them");
+constexpr int kTkCounts = 20;              // passes of the search over 16-bit words, at most
 constexpr int kTkRegion = 16;           // per-thread candidate entries of a register-held row
 static_assert(kTkRegion * kTkThreads * 8 <= kTkSubHists * kTkHistStride * 4, "regions fit the histograms' LDS");
 
-// The candidates of a register-held row (kr: its raw bf16 words, 0xffff past it) from group maxima:
-// bf16 bits compare as signed 16-bit integers wherever the larger value is positive, so a thread's
-// largest word is one packed max per dword, with no key conversion. The k-th largest of the 256
-// maxima of 4 threads each (a binary search on 15 bits over ballots of one wave) is at most the
-// row's k-th largest logit, and about -256 ln(1 - k / 256) logits (56 for k = 50, 177 for 128) reach it
-// when the top logits lie at random; they are found by one more packed max per 16-byte vector,
-// and each counts the larger ones to get its place. False, with nothing written, when the bound is
-// not positive or more than kTkRanked logits reach it (ties, negative rows, top logits that share
-// a few threads): the caller's radix select then does the row. Every thread calls it; same result.
-// Against that select, whose key conversion, counts and byte histogram are 10 passes over the
-// registers: 208 rows of 151,936 logits with a peaked head, top 50, 43 -> 18 us
-// (3.5 TB/s); 24 rows 34 -> 10 us; top 128 of 208 rows 21 us.
-__device__ bool topk_by_maxima(const TopKParams& p, const uint16_t* row, const uint32_t (&kr)[kTkResident][4], int32_t* groups,
-                               uint64_t* cand, int32_t* bound, int32_t* count) {
+// Up to 128 candidates of a register-held row with a vector for every thread. bf16 bits compare as
+// signed 16-bit integers wherever the larger value is positive, so a thread's largest word is one packed max
+// per dword, with no key conversion. The k-th largest of the 256 maxima of 4 threads each (a binary search
+// over ballots of one wave) is at most the row's k-th largest logit, and about -256 ln(1 - k / 256) logits
+// (56 for k = 50, 177 for 128) reach it when the top logits lie at random; they are found by one more
+// packed max per 16-byte vector, and each counts the larger ones to get its place. What that does not settle:
+//   * the k-th maximum is not positive: the words are turned into order-preserving ones (the select's keys,
+//     sign bit flipped, so -0 and +0 tie) and the maxima taken again;
+//   * more than kTkRanked logits reach the bound (top logits that share a few threads): a binary search by
+//     counts over the registers, in which waves without a logit that large take no part, raises it;
+//   * still more do at the k-th logit itself (ties, rows masked to -inf): the larger ones, then as many ties as
+//     are missing, in id order.
+// Bound by the row's load (1,024 threads a CU) and the passes over its registers. us, radix select (which does
+// the other rows: 10 passes, a histogram in LDS where the k-th logit is not near the top) -> here, 208 rows of
+// 151,936: peaked head, top 50 41.4 -> 15.7; log-probabilities 24.8 -> 21.0; 10 finite logits 410 -> 25.8; a 400-logit cluster,
+// top 128 35.0 -> 27.7; 24 rows, peaked 33.8 -> 10.1.
+__global__ __launch_bounds__(kTkThreads) void topk_few_kernel(TopKParams p) {
+  __shared__ int32_t groups[kTkGroups];
+  __shared__ alignas(16) uint64_t cand[kTkRanked + 4];
+  __shared__ int32_t bound, count;
+  __shared__ int32_t counts[kTkCounts];       // of the search's passes
+  __shared__ int32_t ties[2][kTkThreads / 64];
   const int t = threadIdx.x, lane = t & 63;
+  const uint16_t* row = p.logits + int64_t(blockIdx.x) * p.stride;
+  const uint4* rv = reinterpret_cast<const uint4*>(row);
   const int nv = p.vocab >> 3, kk = p.k;
-  const int tail = (nv << 3) + t;  // the logit past the last whole vector that this thread holds
-  const int tail_word = tail < p.vocab ? int(int16_t(row[tail])) : INT16_MIN;
-  i16x2 m = __builtin_bit_cast(i16x2, kr[0][0]);
-#pragma unroll
-  for (int j = 0; j < kTkResident; ++j)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) m = __builtin_elementwise_max(m, __builtin_bit_cast(i16x2, kr[j][e]));
-  int most = max(max(int(m.x), int(m.y)), tail_word);
-  most = max(most, __builtin_amdgcn_update_dpp(0, most, 0xB1, 0xF, 0xF, false));
-  most = max(most, __builtin_amdgcn_update_dpp(0, most, 0x4E, 0xF, 0xF, false));
-  if ((t & 3) == 0) groups[t >> 2] = most;
-  if (t < kTkRanked + 4) cand[t] = 0;  // the last four ranked together may be fewer
-  __syncthreads();
-  if (t < 64) {
-    int g[kTkGroups / 64];
-#pragma unroll
-    for (int i = 0; i < kTkGroups / 64; ++i) g[i] = groups[64 * i + lane];
-    int b = 0;  // the largest bound that kk maxima reach; 0: none that is positive
-    for (int bit = 14; bit >= 0; --bit) {
-      const int c = b | (1 << bit);
-      int n = 0;
-#pragma unroll
-      for (int i = 0; i < kTkGroups / 64; ++i) n += __builtin_popcountll(__ballot(g[i] >= c));
-      if (n >= kk) b = c;
-    }
-    if (t == 0) {
-      *bound = b;
-      *count = 0;
-    }
-  }
-  __syncthreads();
-  const int b = *bound;
-  if (b == 0) return false;
-  auto push = [&](int id, int word) {
-    const int slot = atomicAdd(count, 1);
-    if (slot < kTkRanked) cand[slot] = (uint64_t(uint32_t(word)) << 32) | uint64_t(0xffffffffu - uint32_t(id));
-  };
+  uint32_t kr[kTkResident][4];
 #pragma unroll
   for (int j = 0; j < kTkResident; ++j) {
-    i16x2 v = __builtin_bit_cast(i16x2, kr[j][0]);
+    const int v = t + j * kTkThreads;
+    // slots past the row: a negative NaN, the lowest word and key there is
+    const uint4 w = v < nv ? rv[v] : make_uint4(~0u, ~0u, ~0u, ~0u);
+    kr[j][0] = w.x;
+    kr[j][1] = w.y;
+    kr[j][2] = w.z;
+    kr[j][3] = w.w;
+  }
+  const int tail = (nv << 3) + t;  // the logit past the last whole vector that this thread holds
+  int tail_word = tail < p.vocab ? int(int16_t(row[tail])) : INT16_MIN;
+  if (t < kTkRanked + 4) cand[t] = 0;  // the last four ranked together may be fewer
+  if (t < kTkCounts) counts[t] = 0;
+  if (t == 0) count = 0;
+
+  bool ordered = false;
+  int most, b;  // this thread's largest word, the bound
+  for (;;) {
+    i16x2 m = __builtin_bit_cast(i16x2, kr[0][0]);
 #pragma unroll
-    for (int e = 1; e < 4; ++e) v = __builtin_elementwise_max(v, __builtin_bit_cast(i16x2, kr[j][e]));
-    if (max(int(v.x), int(v.y)) >= b) {
+    for (int j = 0; j < kTkResident; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const i16x2 w = __builtin_bit_cast(i16x2, kr[j][e]);
-        const int id = 8 * (t + j * kTkThreads) + 2 * e;
-        if (int(w.x) >= b) push(id, w.x);
-        if (int(w.y) >= b) push(id + 1, w.y);
+      for (int e = 0; e < 4; ++e) m = __builtin_elementwise_max(m, __builtin_bit_cast(i16x2, kr[j][e]));
+    most = max(max(int(m.x), int(m.y)), tail_word);
+    int g4 = most;
+    g4 = max(g4, __builtin_amdgcn_update_dpp(0, g4, 0xB1, 0xF, 0xF, false));
+    g4 = max(g4, __builtin_amdgcn_update_dpp(0, g4, 0x4E, 0xF, 0xF, false));
+    if ((t & 3) == 0) groups[t >> 2] = g4;
+    __syncthreads();
+    if (t < 64) {
+      int g[kTkGroups / 64];
+#pragma unroll
+      for (int i = 0; i < kTkGroups / 64; ++i) g[i] = groups[64 * i + lane];
+      int at = INT16_MIN;  // the largest word that kk maxima reach
+      for (int bit = 15; bit >= 0; --bit) {
+        const int c = at + (1 << bit);
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < kTkGroups / 64; ++i) n += __builtin_popcountll(__ballot(g[i] >= c));
+        if (n >= kk) at = c;
+      }
+      if (t == 0) bound = at;
+    }
+    __syncthreads();
+    b = bound;
+    if (b > 0 || ordered) break;
+    ordered = true;
+#pragma unroll
+    for (int j = 0; j < kTkResident; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) kr[j][e] = bf16x2_keys(kr[j][e]) ^ 0x80008000u;
+    tail_word = tail < p.vocab ? int(int16_t(bf16_key(row[tail]) ^ 0x8000u)) : INT16_MIN;
+  }
+
+  // Every logit whose word is at least `from` (above the lowest word) into cand, in any order; a thread that
+  // meets the end of the room stops, so that count says no more than that there are too many.
+  auto entry = [&](int id, int word) {
+    return (uint64_t(uint32_t(word + 0x8000)) << 32) | uint64_t(0xffffffffu - uint32_t(id));
+  };
+  auto collect = [&](int from) {
+    bool room = true;
+    auto push = [&](int id, int word) {
+      const int slot = atomicAdd(&count, 1);
+      if (slot < kTkRanked)
+        cand[slot] = entry(id, word);
+      else
+        room = false;
+    };
+#pragma unroll
+    for (int j = 0; j < kTkResident; ++j) {
+      i16x2 v = __builtin_bit_cast(i16x2, kr[j][0]);
+#pragma unroll
+      for (int e = 1; e < 4; ++e) v = __builtin_elementwise_max(v, __builtin_bit_cast(i16x2, kr[j][e]));
+      if (max(int(v.x), int(v.y)) >= from && room) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const i16x2 w = __builtin_bit_cast(i16x2, kr[j][e]);
+          const int id = 8 * (t + j * kTkThreads) + 2 * e;
+          if (int(w.x) >= from) push(id, w.x);
+          if (int(w.y) >= from) push(id + 1, w.y);
+        }
       }
     }
-  }
-  if (tail_word >= b) push(tail, tail_word);
+    if (tail_word >= from) push(tail, tail_word);
+  };
+  if (b > INT16_MIN) collect(b);
   __syncthreads();
-  const int n = *count;
-  if (n > kTkRanked) return false;
+  int n = b > INT16_MIN ? count : kTkRanked + 1;  // (a row of 8,192 logits or more reaches the lowest word)
+  if (n > kTkRanked) {
+    // lo: more than kTkRanked logits reach it. hi: n_hi < kk do.
+    int top = INT16_MIN;
+#pragma unroll
+    for (int i = 0; i < kTkGroups / 64; ++i) top = max(top, groups[64 * i + lane]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) top = max(top, __shfl_xor(top, off));
+    int lo = b, hi = __builtin_amdgcn_readfirstlane(top) + 1, n_hi = 0, pass = 0;
+    bool settled = false;
+    while (hi - lo > 1) {
+      const int mid = pass == 0 ? lo + 1 : lo + (hi - lo) / 2;  // first: are all but kk at most of them ties?
+      int c = 0;
+      if (most >= mid) {
+        const short m = static_cast<short>(mid);
+        const i16x2 thr = {m, m};
+        i16x2 below = {0, 0};  // -1 for each smaller word (slots past the row always are)
+#pragma unroll
+        for (int j = 0; j < kTkResident; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            below += __builtin_elementwise_sub_sat(__builtin_bit_cast(i16x2, kr[j][e]), thr) >> 15;
+        c = 8 * kTkResident + int(below.x) + int(below.y) + (tail_word >= mid);
+      }
+      if (__ballot(c != 0) != 0) {
+        c = wave_sum_int(c);
+        if (lane == 0) atomicAdd(&counts[pass], c);
+      }
+      __syncthreads();
+      c = counts[pass++];
+      if (c < kk) {
+        hi = mid;
+        n_hi = c;
+      } else {
+        lo = mid;
+        if (c <= kTkRanked) {
+          settled = true;
+          break;
+        }
+      }
+    }
+    __syncthreads();  // (every thread has read count)
+    if (t == 0) count = 0;
+    __syncthreads();
+    if (settled || n_hi > 0) collect(settled ? lo : hi);
+    if (!settled) {
+      // n_hi larger ones; ties of the k-th logit behind them, a vector of every thread at a time (there are more
+      // than kTkRanked - kk ties, so those in whole vectors suffice)
+      int have = n_hi;
+      for (int j = 0; j * kTkThreads < nv && have < kk; ++j) {
+        const int v = t + j * kTkThreads;
+        uint32_t w[4] = {0, 0, 0, 0};
+        int c = 0;
+        if (v < nv) {
+          const uint4 q = rv[v];
+          w[0] = q.x, w[1] = q.y, w[2] = q.z, w[3] = q.w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (ordered) w[e] = bf16x2_keys(w[e]) ^ 0x80008000u;
+            const i16x2 x = __builtin_bit_cast(i16x2, w[e]);
+            c += (int(x.x) == lo) + (int(x.y) == lo);
+          }
+        }
+        int sum = c;  // of this lane's and the lower lanes'
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const int o = __shfl_up(sum, off);
+          if (lane >= off) sum += o;
+        }
+        if (lane == 63) ties[j & 1][t >> 6] = sum;
+        __syncthreads();
+        int at = have + sum - c;
+#pragma unroll
+        for (int i = 0; i < kTkThreads / 64; ++i) {
+          if (i < (t >> 6)) at += ties[j & 1][i];
+          have += ties[j & 1][i];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const i16x2 x = __builtin_bit_cast(i16x2, w[e]);
+          if (v < nv && int(x.x) == lo && at < kk) cand[at] = entry(8 * v + 2 * e, lo);
+          at += v < nv && int(x.x) == lo;
+          if (v < nv && int(x.y) == lo && at < kk) cand[at] = entry(8 * v + 2 * e + 1, lo);
+          at += v < nv && int(x.y) == lo;
+        }
+      }
+    }
+    __syncthreads();
+    n = settled ? count : kk;
+    if (t < 4) cand[n + t] = 0;
+    __syncthreads();
+  }
   if (t < n) {
     const uint64_t own = cand[t];  // larger word first, then the lower id
     int place = 0;
@@ -299,11 +435,11 @@ __device__ bool topk_by_maxima(const TopKParams& p, const uint16_t* row, const u
       place += (a.x > own) + (a.y > own) + (c.x > own) + (c.y > own);
     }
     if (place < kk) {
-      p.values[int64_t(blockIdx.x) * p.k + place] = uint16_t(own >> 32);
-      p.ids[int64_t(blockIdx.x) * p.k + place] = int64_t(0xffffffffu - uint32_t(own)) + p.vocab_start;
+      const uint32_t id = 0xffffffffu - uint32_t(own);
+      p.values[int64_t(blockIdx.x) * p.k + place] = ordered ? row[id] : uint16_t(uint32_t(own >> 32) - 0x8000u);
+      p.ids[int64_t(blockIdx.x) * p.k + place] = int64_t(id) + p.vocab_start;
     }
   }
-  return true;
 }
 
 template <bool kVec>
@@ -311,7 +447,7 @@ __global__ __launch_bounds__(kTkThreads) void topk_candidates_kernel(TopKParams 
   __shared__ uint32_t hist[kTkSubHists][kTkHistStride];
   __shared__ uint32_t bins[256];
   __shared__ uint32_t bin_part[4][256];
-  __shared__ alignas(16) uint64_t cand[kTkCandCap];
+  __shared__ uint64_t cand[kTkCandCap];
   __shared__ int32_t sel[6];  // threshold key, count above, ties needed, candidates written, ties present,
                               // a region overflowed
   __shared__ int32_t tie_scan[kTkThreads];
@@ -324,8 +460,8 @@ __global__ __launch_bounds__(kTkThreads) void topk_candidates_kernel(TopKParams 
   const int V = p.vocab;
   const int kk = min(p.k, V);
 
-  // Rows of up to kTkResident vectors per thread are read once: their logits, then their keys,
-  // stay in registers (two 16-bit values per dword) for all passes.
+  // Rows of up to kTkResident vectors per thread are read once: their keys stay in
+  // registers (two 16-bit keys per dword) for all passes.
   uint32_t kr[kTkResident][4];
   const bool resident = kVec && (V >> 3) <= kTkResident * kTkThreads;
   if (resident) {
@@ -337,17 +473,11 @@ __global__ __launch_bounds__(kTkThreads) void topk_candidates_kernel(TopKParams 
       // slots past the row hold raw 0xffff (a negative NaN) in both halves, whose key is 0:
       // below every threshold of the search, never its maximum
       const uint4 w = v < nv ? rv[v] : make_uint4(~0u, ~0u, ~0u, ~0u);
-      kr[j][0] = w.x;
-      kr[j][1] = w.y;
-      kr[j][2] = w.z;
-      kr[j][3] = w.w;
+      kr[j][0] = bf16x2_keys(w.x);
+      kr[j][1] = bf16x2_keys(w.y);
+      kr[j][2] = bf16x2_keys(w.z);
+      kr[j][3] = bf16x2_keys(w.w);
     }
-    // (a vector for every thread, so that every group has a maximum)
-    if (p.k <= kTkMaximaK && nv >= kTkThreads && topk_by_maxima(p, row, kr, tie_scan, cand, &sel[0], &sel[3])) return;
-#pragma unroll
-    for (int j = 0; j < kTkResident; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) kr[j][e] = bf16x2_keys(kr[j][e]);
   }
   // f(i, key) over the row: from registers, else 16-byte loads (8 logits, four in flight per
   // thread) when rows are 16-byte aligned, else element loads
@@ -1026,7 +1156,12 @@ extern "C" int aspire_topk_candidates(const void* logits, int64_t stride, int32_
   TopKParams p{static_cast<const uint16_t*>(logits), stride, vocab, top_k, vocab_start,
                static_cast<uint16_t*>(values), ids};
   const bool vec = (reinterpret_cast<uintptr_t>(logits) & 15) == 0 && stride % 8 == 0;
-  if (vec)
+  // group maxima for up to 128 candidates of rows that give every thread of a workgroup a vector and stay in
+  // its registers; the radix select for the others
+  const int nv = vocab >> 3;
+  if (vec && top_k <= kTkMaximaK && nv >= kTkThreads && nv <= kTkResident * kTkThreads)
+    hipLaunchKernelGGL(topk_few_kernel, dim3(rows), dim3(kTkThreads), 0, static_cast<hipStream_t>(stream), p);
+  else if (vec)
     hipLaunchKernelGGL(topk_candidates_kernel<true>, dim3(rows), dim3(kTkThreads), 0, static_cast<hipStream_t>(stream), p);
   else
     hipLaunchKernelGGL(topk_candidates_kernel<false>, dim3(rows), dim3(kTkThreads), 0, static_cast<hipStream_t>(stream), p);

@@ -87,8 +87,8 @@ def test_topk_candidates_paths(gpu, case):
 @pytest.mark.parametrize("vocab,k", [(8192, 1), (8192, 128), (8199, 50), (8191, 50), (151936, 128), (155651, 100)])
 @pytest.mark.parametrize("case", ["random", "few_positive", "ties_512", "ties_513", "signed_zeros", "infinities"])
 def test_topk_by_group_maxima(gpu, vocab, k, case):
-    """Rows the group maxima settle and rows they leave to the radix select: the smallest and largest
-    register-held row, a tail past the last whole vector, fewer positive logits than k, exactly as many
+    """Rows that the group maxima settle and rows where more logits reach their bound than are ranked: the smallest
+    and largest register-held row, one that is left to the radix select, a tail past the last whole vector, fewer positive logits than k, exactly as many
     ties at the k-th logit as are ranked by counting and one more, zeros of both signs at the k-th
     place, infinities."""
     say("topk by maxima", vocab, k, case)
@@ -115,6 +115,46 @@ def test_topk_by_group_maxima(gpu, vocab, k, case):
     ref_v, ref_i = osamp.topk_candidates(x, k, 11)
     assert torch.equal(ids.cpu(), ref_i)
     assert torch.equal(vals.cpu().view(torch.int16), ref_v.view(torch.int16))
+
+
+@pytest.mark.parametrize("vocab,k", [(8192, 1), (8199, 128), (30005, 50), (151936, 20), (155655, 128)])
+@pytest.mark.parametrize("case", ["log_probs", "masked_few", "masked_all", "cluster", "crowded", "sparse_ties", "lowest"])
+def test_topk_where_the_bound_does_not_settle_it(gpu, vocab, k, case):
+    """Rows without positive logits, masked to -inf up to a few or altogether, with the top logits in a few threads,
+    with more logits at the bound than are ranked at once (distinct and tied), and a row of the lowest word there is."""
+    say("topk unsettled", vocab, k, case)
+    g = torch.Generator().manual_seed(vocab * 3 + k)
+    x = torch.randn(3, vocab, generator=g) * 2
+    at = torch.randperm(vocab, generator=g)
+    if case == "log_probs":
+        x = torch.log_softmax(x, dim=-1)
+    elif case == "masked_few":
+        keep = x[:, at[: k // 2 + 1]] + 1
+        x[:] = float("-inf")
+        x[:, at[: k // 2 + 1]] = keep
+    elif case == "masked_all":
+        x[:] = float("-inf")
+        x[1, vocab - 1] = 0.0                # the tail, and a zero of each sign
+        x[2, vocab // 2], x[2, vocab // 2 + 1] = -0.0, 0.0
+    elif case == "cluster":                  # 700 neighbours, the last of the row among them
+        x[:, -700:] += 40
+    elif case == "crowded":
+        x[:, : 8 * 900] = 30 + 4 * torch.rand(3, 8 * 900, generator=g)
+    elif case == "sparse_ties":              # the k-th is one of 600 ties spread over the row, below k - 1 larger ones
+        x = x.clamp(max=3.0)
+        x[:, at[:600]] = 5.0
+        x[:, at[600 : 599 + k]] = 6 + torch.rand(3, k - 1, generator=g)
+    x = x.to(torch.bfloat16)
+    if case == "lowest":
+        x.view(torch.int16)[:] = -1          # a negative NaN, as the slots past the row hold
+        x[1, 5::97] = float("-inf")
+    vals, ids = local_topk_candidates(x.to(gpu), k, 11)
+    keys = x.view(torch.int16).int()
+    keys = torch.where(keys == -32768, 0, keys)
+    keys = torch.where(keys < 0, keys ^ 0x7FFF, keys)      # in the order of the values
+    ref = torch.stack([torch.from_numpy(np.lexsort((np.arange(vocab), -r.numpy()))[:k]) for r in keys])
+    assert torch.equal(ids.cpu() - 11, ref)
+    assert torch.equal(vals.cpu().view(torch.int16), x.view(torch.int16).gather(1, ref))
 
 
 def test_topk_by_group_maxima_places_nan_as_the_select_does(gpu):
