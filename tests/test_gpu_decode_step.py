@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from aspire_amd import linear as lin
 from aspire_amd.attention.page_list import build_head_page_lists
 from aspire_amd.decode_step import (DecodeWeights, MixedDecodeStep, ModelShape, add_rms_norm, alloc_kv_caches,
                                     argmax_rows, silu_mul)
@@ -238,6 +239,48 @@ def test_decode_step_graph_replays_match_eager(gpu, shape):
         assert torch.equal(glogits, e_logits), f"replay {i} logits"
         assert torch.equal(step.selector.selected, e_sel), f"replay {i} selection"
         _ = torch.randn(1000, device=gpu).sum().item()   # eager work between replays
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_small_decode_step_on_library_products(gpu, shape, monkeypatch):
+    """The steps past linear.MAX_ROWS tokens (library products, SwiGLU as a launch of its own, bf16 projections into
+    the add + norm and the q/k preparation), here at the small step's size: against the oracle, and replayed."""
+    monkeypatch.setattr(lin, "MAX_ROWS", 0)
+    test_small_decode_step_matches_oracle(gpu, shape)
+    test_decode_step_graph_replays_match_eager(gpu, shape)
+
+
+@pytest.mark.parametrize("tokens", [128, 129, 224, 225])
+def test_decode_step_at_the_edges_of_its_dispatch(gpu, tokens, monkeypatch):
+    """Both sides of HEAD_ROWS and linear.MAX_ROWS: which products run, and the logits against a step whose products
+    are all the library's (bf16 roundings through four layers: the oracle test's 1% of the mean |logit|)."""
+    say("decode step dispatch", tokens)
+    ql = np.full(tokens // 5, 5)
+    ql[: tokens - int(ql.sum())] += 1
+    ctx = 20 + (np.arange(len(ql)) * 37) % 300
+    n_pages = (ctx + 15) // 16
+    table, pool = random_block_table(n_pages, seed=9, pool_pages=int(n_pages.sum()))
+    logits, calls = [], []
+    real = lin.linear, lin.linear_partials
+    for library in (False, True):
+        if library:
+            monkeypatch.setattr(lin, "MAX_ROWS", 0)
+        w = DecodeWeights(SMALL, gpu, seed=9)
+        caches = alloc_kv_caches(SMALL, pool, gpu, seed=9)
+        step = MixedDecodeStep(w, caches, ctx, ql, np.zeros(len(ql), bool), torch.from_numpy(table), budget=8,
+                               refresh_layer=2, seed=9)
+        assert step.T == tokens
+        count = {"linear": 0, "partials": 0}
+        monkeypatch.setattr(lin, "linear", lambda *a, **k: (count.update(linear=count["linear"] + 1), real[0](*a, **k))[1])
+        monkeypatch.setattr(lin, "linear_partials",
+                            lambda *a: (count.update(partials=count["partials"] + 1), real[1](*a))[1])
+        step.forward()
+        logits.append(step.logits.float().cpu())
+        calls.append((count["linear"], count["partials"]))
+    layers = SMALL.n_layer
+    assert calls[0] == ((layers + (tokens <= 128), 3 * layers) if tokens <= 224 else (0, 0)) and calls[1] == (0, 0)
+    a, b = logits
+    assert (a - b).abs().mean() <= 0.01 * b.abs().mean() and (a - b).abs().max() <= 0.05 * b.abs().max()
 
 
 @pytest.mark.parametrize("vocab", [1, 7, 8, 8191, 8200, 40960, 40969, 151936])

@@ -15,6 +15,10 @@ pytestmark = pytest.mark.gpu
 ROWS = [1, 16, 17, 32, 33, 64, 65, 100, 128, 129, 208, 224]
 
 
+# slabs up to 16, 128 and 224 rows, where a case is there for them
+SPLITS = {(1056, 2432): (8, 8, 8), (6144, 4096): (3, 5, 4), (4096, 12288): (4, 8, 5)}
+
+
 def close_sum(got, x, w, ref, ulps=0.0):
     """Products of bf16 are exact in fp32; a sum of K of them in fp32, in any order, is within
     K * 2^-24 of sum |x w| (gamma_K of the standard bound), plus ``ulps`` roundings to bf16 (8 significant bits: 2^-8 of the value each)."""
@@ -31,9 +35,16 @@ def operands(rows, n, k, gpu, pad=0):
 
 
 @pytest.mark.parametrize("rows", ROWS)
-@pytest.mark.parametrize("n,k,pad", [(32, 128, 0), (96, 256, 8), (4128, 384, 0), (25600, 128, 16), (12320, 640, 0)])
+@pytest.mark.parametrize("n,k,pad", [
+    (32, 128, 0), (96, 256, 8), (4128, 384, 0), (25600, 128, 16), (12320, 640, 0),
+    (1056, 2432, 0),    # 8 splits of 38 steps: unequal ones, rings that wrap a few times
+    (6144, 4096, 0),    # 64-row tiles in 3 splits, 128-row in 5, 96-row (past 128 rows) in 4
+    (4096, 12288, 8),   # 4, 8 and 5 splits, long walks over k
+    (16480, 640, 8),    # 96-row tiles past 64 rows for both outputs, the last one past the weight's end
+    (24640, 1152, 0),   # 128-row tiles from 33 rows on
+])
 def test_linear_and_partials(gpu, rows, n, k, pad):
-    """One k step, tiles that end past the last weight row, every tile width the chooser takes (few and
+    """One k step and many, tiles that end past the last weight row, every tile width the chooser takes (few and
     many tiles), row strides longer than k; both outputs, nothing written beside them."""
     say("linear", rows, n, k, pad)
     x, w = operands(rows, n, k, gpu, pad)
@@ -43,6 +54,8 @@ def test_linear_and_partials(gpu, rows, n, k, pad):
     close_sum(out[:rows, :n], x, w, ref, ulps=1)
     assert (out[rows:] == 7).all() and (out[:, n:] == 7).all()
     s = linear_splits(rows, n, k)
+    if (n, k) in SPLITS:
+        assert s == SPLITS[n, k][0 if rows <= 16 else 1 if rows <= 128 else 2]
     ws = torch.full((s * rows * n + 64,), 7.0, device=gpu)
     parts = linear_partials(x, w, ws)
     assert parts.shape == (s, rows, n) and (ws[s * rows * n :] == 7).all()
@@ -50,7 +63,13 @@ def test_linear_and_partials(gpu, rows, n, k, pad):
 
 
 @pytest.mark.parametrize("rows", ROWS)
-@pytest.mark.parametrize("n,k", [(16, 128), (1040, 512), (12304, 256)])
+@pytest.mark.parametrize("n,k", [
+    (16, 128), (1040, 512), (12304, 256),
+    (1040, 2432),       # 64-row tiles, rings that wrap at every row class
+    (8224, 2176),       # 96-row tiles past 64 rows, the last one past the weight's end
+    (13648, 2304),      # 128-row tiles from 17 to 128 rows
+    (12288, 4096),
+])
 def test_linear_swiglu(gpu, rows, n, k):
     say("linear swiglu", rows, n, k)
     x, w = operands(rows, 2 * n, k, gpu)
