@@ -18,6 +18,7 @@
 //     (a, b) -> (a cos - b sin, b cos + a sin) in fp32, rounded to bf16;
 //   * append: the row / slot rule of the plain append (append_locate).
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 
@@ -57,6 +58,7 @@ struct RopeParams {
 // Head slots of one wave pass: 4 groups of 16 lanes, one head each.
 constexpr int kRopeHeads = 4;
 constexpr int kRopeWaves = 4;   // waves per workgroup
+constexpr int64_t kRopeMaxWaves = 2816;  // 11 a CU: waves past that cost more than the passes they spare
 
 __device__ __forceinline__ float lo_bf(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi_bf(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
@@ -119,7 +121,9 @@ __device__ __forceinline__ void round_pair(float& x, float& y) {
 // heads (1.2 TB/s, bound by the sincosf and address arithmetic) where this takes 48 us (4.2 TB/s);
 // 208 tokens 6.3 -> 4.8 us.
 // kSum: the inputs are the slabs of a split projection; q is written to p.q, nothing is read from it.
-template <bool kWide, bool kSum>
+// kNorm (not with kSum, which looks) / kAppend: with the norm weights / a cache. The rotation alone is 0.15 us
+// shorter without their code.
+template <bool kWide, bool kSum, bool kNorm, bool kAppend>
 __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(RopeParams p, int total_tokens, int wpt_log2) {
   __shared__ float2 rot[kRopeWaves][kPairs];
   const int lane = threadIdx.x & 63;
@@ -129,9 +133,9 @@ __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(Ro
   const int part = unit & ((1 << wpt_log2) - 1);
   if (tok >= total_tokens) return;
   const int j = lane & 15, grp = lane >> 4;
-  const bool permute = p.permute != 0, norm = p.q_w != nullptr;
+  const bool norm = kSum ? p.q_w != nullptr : kNorm, permute = norm && p.permute != 0;
   const int n_qk = p.hq + p.hkv;
-  const int n_all = p.cache != nullptr && p.v != nullptr ? n_qk + p.hkv : n_qk;
+  const int n_all = kAppend && p.v != nullptr ? n_qk + p.hkv : n_qk;
   const int step = kRopeHeads << wpt_log2;
 
   // a head's words: q / k dims for the rotation, 16 bytes of v for the copy
@@ -145,7 +149,7 @@ __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(Ro
       w = load_lane_dims<kWide>(p.q + int64_t(tok) * p.q_st + int64_t(h) * p.q_sh, j, permute);
     } else if (h < n_qk) {
       w = load_lane_dims<kWide>(p.k + int64_t(tok) * p.k_st + int64_t(h - p.hq) * p.k_sh, j, permute);
-    } else if (h < n_all) {
+    } else if (kAppend && h < n_all) {
       w = *reinterpret_cast<const uint4*>(p.v + int64_t(tok) * p.v_st + int64_t(h - n_qk) * p.v_sh + 8 * j);
     }
     return w;
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(Ro
     const int begin = p.indptr[b], end = p.indptr[b + 1];
     if (tok < end) {
       pos = wave_uniform(p.offsets[b] + tok - begin);
-      if (p.cache != nullptr && b < p.num_seq) {
+      if (kAppend && b < p.num_seq) {
         const int first = p.page_indptr[b];
         const int pages = p.page_indptr[b + 1] - first;
         const int seq_len = max(pages - 1, 0) * p.page_size + p.last_page_len[b];
@@ -198,7 +202,7 @@ __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(Ro
     const uint4 w = cur;
     cur = next;
     if (h >= n_qk) {
-      if (h < n_all && page_k != nullptr)
+      if (kAppend && h < n_all && page_k != nullptr)
         *reinterpret_cast<uint4*>(page_k + p.c_skv + int64_t(h - n_qk) * p.c_sh + 8 * j) = w;
       continue;
     }
@@ -239,7 +243,7 @@ __global__ __launch_bounds__(64 * kRopeWaves) void qk_norm_rope_append_kernel(Ro
         for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(row + 8 * j + 2 * e) = o[e];
       }
     }
-    if (!is_q && page_k != nullptr)
+    if (kAppend && !is_q && page_k != nullptr)
       *reinterpret_cast<uint4*>(page_k + int64_t(h - p.hq) * p.c_sh + 8 * j) = make_uint4(o[0], o[1], o[2], o[3]);
   }
 }
@@ -339,18 +343,29 @@ int prepare_qkv(const aspire_rope_args* a, const float* partials, int32_t splits
   const bool wide = aligned(a->q, 16) && aligned(a->k, 16) && aligned(p.q_w, 8) && aligned(p.k_w, 8) &&
                     a->q_stride_t % 8 == 0 && a->q_stride_h % 8 == 0 && a->k_stride_t % 8 == 0 &&
                     a->k_stride_h % 8 == 0;
-  // Waves per token: enough waves to hide the look-up's latency, then as few as share one sincosf.
-  // us at 16 / 8 / 4 waves (32 q / 8 kv heads): 1 token 3.4 / 4.0 / 4.6, 16: 3.5 / 4.1 / 4.8, 80:
-  // 3.9 / 4.3 / 4.9, 208: 5.0 / 4.8 / 5.2, 512: 7.9 / 7.0 / 6.4, 8,192: 81 / 62 / 48; with 16 / 8
-  // heads 80: 3.9 / 3.6 / 4.2, 304: 5.5 / 4.4 / 4.7, 512: 7.7 / 5.1 / 5.1.
-  const int wpt_log2 = a->total_tokens <= 32 ? 4 : a->total_tokens <= 256 ? 3 : 2;
+  // Waves per token: one for each quad of heads, so that a token is done in one pass of its waves, as
+  // long as that keeps the launch within kRopeMaxWaves; past it as many as fit, then 4, which share one sincosf
+  // (8,192 tokens: 81 / 62 / 48 us at 16 / 8 / 4). us at 4 / 8 / 16 / 32 waves, 32 q / 8 kv heads (12 quads):
+  // 33 tokens 5.7 / 5.0 / 4.4 / 4.6, 160: 5.9 / 5.5 / 5.5 / 6.5, 208: 6.0 / 5.7 / 5.9 / 7.6, 400: 6.9 / 7.0 / 7.6;
+  // 64 / 8 (20): 33: 7.1 / 5.7 / 5.0 / 4.6, 104: 7.3 / 5.9 / 5.6 / 5.8, 300: 8.8 / 7.7 / 8.0; 16 / 8 (8): 33: 5.0 / 4.4 /
+  // 4.4, 300: 5.7 / 5.4 / 6.4. (One wave a head, as it was once, takes 4.4, 6.0, 7.0 and 10.0 in the first row's places.)
+  const int quads = (a->num_qo_heads + a->num_kv_heads * (p.cache && p.v ? 2 : 1) + kRopeHeads - 1) / kRopeHeads;
+  int wpt_log2 = 2;
+  while ((1 << wpt_log2) < quads && (int64_t(a->total_tokens) << (wpt_log2 + 1)) <= kRopeMaxWaves) ++wpt_log2;
   ASPIRE_CHECK_ARG(partials == nullptr || (p.cache != nullptr && wide && aligned(partials, 16) && splits >= 1 && !a->write_k),
                    "partials need a cache, 16-byte aligned slabs and q rows, and write_k 0");
   const int64_t units = int64_t(a->total_tokens) << wpt_log2;
   const dim3 grid(unsigned((units + kRopeWaves - 1) / kRopeWaves));
-  const auto kernel = p.partials ? qk_norm_rope_append_kernel<true, true>
-                      : wide     ? qk_norm_rope_append_kernel<true, false>
-                                 : qk_norm_rope_append_kernel<false, false>;
+  const auto pick = [&](auto kWide, auto kNorm) {
+    return p.cache ? qk_norm_rope_append_kernel<kWide(), false, kNorm(), true>
+                   : qk_norm_rope_append_kernel<kWide(), false, kNorm(), false>;
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  const bool norm = p.q_w != nullptr;
+  const auto kernel = p.partials ? qk_norm_rope_append_kernel<true, true, true, true>
+                      : wide     ? (norm ? pick(yes, yes) : pick(yes, no))
+                                 : (norm ? pick(no, yes) : pick(no, no));
   hipLaunchKernelGGL(kernel, grid, dim3(64 * kRopeWaves), 0, static_cast<hipStream_t>(stream), p, a->total_tokens,
                      wpt_log2);
   ASPIRE_CHECK_LAUNCH();

@@ -93,12 +93,15 @@ def pairs_close(got: torch.Tensor, ref: torch.Tensor):
 
 
 @pytest.mark.parametrize("hq,hkv,lens,width", [
-    (32, 8, [1], 128),                       # the smallest call: 16 waves a token
+    (32, 8, [1], 128),                       # the smallest call
     (7, 3, [5, 0, 26], 128),                 # heads that fill no quad; 31 tokens, an empty row
-    (16, 2, [33], 136),                      # 33 tokens: 8 waves a token; strided heads
+    (16, 2, [33], 136),                      # 8 waves a token, more than quads; strided heads
     (6, 6, [100, 156], 130),                 # head rows 4-byte but not 8-byte aligned: the narrow loads
-    (32, 8, [257], 128),                     # 257 tokens: 4 waves a token, a last workgroup of its own
+    (32, 8, [257], 128),                     # a last workgroup with waves past the tokens
     (5, 1, [300, 1, 900], 128),
+    (64, 8, [3, 28], 128),                   # 20 quads: 32 waves a token, some without heads
+    (40, 16, [86], 132),                     # 88 tokens with the padding: the most that 32 waves each are launched for
+    (40, 16, [87], 128),                     # and one more: 16 waves, two passes
 ])
 @pytest.mark.parametrize("norm", [True, False])
 def test_fused_edges_match_oracle(gpu, hq, hkv, lens, width, norm):
