@@ -113,6 +113,8 @@ struct PrefillParams {
   float* part_lse;    // [slots][num_kv_heads][kPfBlockRows], base 2
 };
 
+// kUnits: takes p.units; else whole blocks, the last one first.
+template <bool kUnits>
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfWavesPerEu))) void prefill_kernel(
     PrefillParams p) {
   __shared__ uint4 stg0[kPfStage];
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
   const int g = wave_uniform(int(blockIdx.x) % hkv);
   const int unit = wave_uniform(int(blockIdx.x) / hkv);
   int4 piece = make_int4(p.total_blocks - 1 - unit, 0, 0x7fffffff, -1);
-  if (p.units != nullptr) piece = p.units[unit];
+  if (kUnits) piece = p.units[unit];
   const int blk = wave_uniform(piece.x);
   int lo = 0, hi = p.num_rows - 1, b = 0;
   while (lo <= hi) {
@@ -167,8 +169,8 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
   const int blk_last = p.causal ? min(shift + tok0 + ntok - 1, kv_len - 1) : kv_len - 1;
   const int blk_pages = blk_last >= 0 ? blk_last / kPage + 1 : 0;
   // this workgroup's steps (a piece's end may lie past the block's last step: the last piece takes them all)
-  const int begin = wave_uniform(piece.y);
-  const int steps = wave_uniform(min((blk_pages + 1) / 2, piece.z));
+  const int begin = kUnits ? wave_uniform(piece.y) : 0;
+  const int steps = wave_uniform(kUnits ? min((blk_pages + 1) / 2, piece.z) : (blk_pages + 1) / 2);
   const int vlim = wave_uniform(min(kv_len, blk_pages * kPage));
   const int w_last = wave_uniform(rows > 0 ? (p.causal ? min(shift + wt0 + wn - 1, kv_len - 1) : kv_len - 1) : -1);
   const int w_min_limit = wave_uniform(p.causal ? min(shift + wt0, kv_len - 1) : kv_len - 1);
@@ -431,7 +433,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kPfW
     const int ti = row / G;
     const int head = g * G + (row - ti * G);
     const int token = q0 + wt0 + ti;
-    if (piece.w >= 0) {
+    if (kUnits && piece.w >= 0) {
       const int64_t slot = (int64_t(piece.w) * hkv + g) * kPfBlockRows + wave * kPfRows + row;
       float* dst = p.part_o + slot * kHeadDim;
 #pragma unroll
@@ -762,7 +764,8 @@ int prefill_launch(const aspire_prefill_args* a, const int32_t* units, int32_t n
                      "bad units, or partials smaller than slots * num_kv_heads * block rows * 129 floats");
   ASPIRE_CHECK_ARG(int64_t(num_units) * a->num_kv_heads < (int64_t(1) << 31), "too many units");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(prefill_kernel, dim3(num_units * a->num_kv_heads), dim3(kPfThreads), 0, s, p);
+  const auto kernel = units != nullptr ? prefill_kernel<true> : prefill_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(num_units * a->num_kv_heads), dim3(kPfThreads), 0, s, p);
   if (units != nullptr && num_merges > 0)
     hipLaunchKernelGGL(prefill_merge_kernel, dim3(num_merges * a->num_kv_heads * (kPfBlockRows / 16)), dim3(256), 0, s,
                        p, reinterpret_cast<const int4*>(merges));

@@ -346,3 +346,21 @@ def test_prefill_without_room_for_partials_runs_whole_blocks(gpu, monkeypatch):
                                        step.kv_indices.cpu(), step.kv_len_host, num_kv_heads=8, causal=True)
     attn_close(out[:T], ref_out[:T])
     assert (lse[:T].cpu() - ref_lse[:T]).abs().max() < 2e-3
+
+
+@pytest.mark.parametrize("rows,prefix,listed", [(8, 0, False), (20, 0, True), (36, 0, False), (36, 430, True)])
+def test_prefill_lists_whole_blocks_where_that_pays(gpu, rows, prefix, listed):
+    """A block a CU, two, and more than four of short and of longer blocks: with and without a list, against the oracle."""
+    say("prefill list", rows, prefix)
+    q_len = [68 + (i * 37) % 52 for i in range(rows)]
+    ctx = [n + prefix for n in q_len]
+    step = build_step(hq=32, hkv=32, ctx_len=ctx, q_len=q_len, is_draft=[0] * rows, draft_budget=0, seed=44, device=gpu)
+    w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(1, device=gpu), "NHD")
+    w.plan(step.qo_indptr[:-1], step.kv_indptr[:-1], step.kv_indices, step.last_page_len[:-1], 32, 32, 128, PAGE, causal=True)
+    assert w._pf["slots"] == 0 and (w._pf["units"] is not None) == listed
+    out, lse = w.run(step.q, step.cache, return_lse=True)
+    ref_out, ref_lse = paged_attention(step.q.cpu(), step.cache.cpu(), step.qo_indptr_host, step.kv_indptr_host,
+                                       step.kv_indices.cpu(), step.kv_len_host, num_kv_heads=32, causal=True)
+    T = step.total_tokens
+    attn_close(out[:T], ref_out[:T])
+    assert (lse[:T].cpu() - ref_lse[:T]).abs().max() < 2e-3
