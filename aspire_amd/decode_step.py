@@ -13,10 +13,10 @@ The step follows ``TransformerSparseDraft.unified_forward``
 
 Steps of at most ``linear.MAX_ROWS`` tokens run their projections on the HIP
 library's own kernels (``aspire_amd.linear``): w13 with the SwiGLU step in its
-epilogue, and wqkv, wo and w2 split over K, their fp32 partial sums taken by the
-launch that follows anyway (the q/k preparation, the residual add + norm). Larger
-steps use torch's GEMMs (hipBLASLt), as does the vocabulary projection past
-``HEAD_ROWS`` tokens. The q/k preparation and the append are one launch
+epilogue (where ``linear.swiglu_pays``), and wqkv, wo and w2 split over K, their fp32
+partial sums taken by the launch that follows anyway (the q/k preparation, the
+residual add + norm). Larger steps use torch's GEMMs (hipBLASLt), as does the
+vocabulary projection past ``HEAD_ROWS`` tokens. The q/k preparation and the append are one launch
 (``qk_norm_rope_update_kv``), the attention is ``HolisticAttentionWrapper``, and
 the residual adds, norms and token pick are the row kernels of the HIP library
 (``aspire_add_rms_norm``, ``aspire_argmax_rows``), so a whole step can be
@@ -388,7 +388,7 @@ class MixedDecodeStep:
             raise ValueError("tokens must hold one id per new token")
         self.x = torch.empty(T, shape.dim, dtype=bf, device=dev)
         self.a = torch.empty(T, shape.dim, dtype=bf, device=dev)
-        # q of attention_only (the forward's projections are fresh tensors)
+        # q of attention_only (the forward's projections go to partials and q, or are fresh tensors)
         self.qkv = torch.empty(T, shape.q_size + 2 * shape.kv_size, dtype=bf, device=dev).normal_()
         self.y = torch.empty(T, shape.n_head, shape.head_dim, dtype=bf, device=dev)
         self.act = torch.empty(T, shape.intermediate_size, dtype=bf, device=dev)
@@ -490,7 +490,7 @@ class MixedDecodeStep:
             if capture is not None:
                 capture[f"y{layer}"] = self.y.clone()
             self._add_norm(lw["ffn_norm"], self._project(self.y.view(self.T, s.q_size), lw["wo"]))
-            if lin.supported(self.a, lw["w13"]):
+            if lin.supported(self.a, lw["w13"]) and lin.swiglu_pays(self.T, s.intermediate_size):
                 lin.linear(self.a, lw["w13"], self.act, swiglu=True)
             else:
                 silu_mul(F.linear(self.a, lw["w13"]), self.act)

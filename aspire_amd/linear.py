@@ -28,6 +28,15 @@ def supported(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.shape[1] % 128 == 0 and w.shape[0] % 32 == 0)
 
 
+def swiglu_pays(rows: int, n: int) -> bool:
+    """Whether ``linear(..., swiglu=True)`` is the shorter way to ``n`` columns, against the library's product and
+    ``silu_mul``. Past 128 rows a workgroup holds 48 columns and a CU one workgroup, so more than 256 x 48
+    take a second round. Own over library time at 136 to 224 rows, weights cold: 12,288 columns 0.82 to 0.93
+    (K 2,048 to 5,120), 12,416 1.16 to 1.34, 14,336 1.14 to 1.32, 17,408 1.00 to 1.16, 25,600 1.24 to 1.55; up to 128
+    rows 0.4 to 1.0, but 1.1 for 25,600 x 5,120."""
+    return rows <= 128 or n <= 256 * 48
+
+
 def _check(x, w, what):
     _lib.require_cuda(x, w, what=what)
     if not supported(x, w):
@@ -68,4 +77,4 @@ def linear_partials(x: torch.Tensor, w: torch.Tensor, workspace: torch.Tensor) -
     return workspace.view(-1)[: s * rows * n].view(s, rows, n)
 
 
-__all__ = ["MAX_ROWS", "supported", "linear", "linear_splits", "linear_partials"]
+__all__ = ["MAX_ROWS", "supported", "swiglu_pays", "linear", "linear_splits", "linear_partials"]

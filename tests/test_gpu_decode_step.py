@@ -1,6 +1,8 @@
 """The full decode step's GPU pieces against the CPU oracle: the row kernels, the per-head
 page lists, a small model step end to end, and the step recorded in a HIP graph."""
 
+from dataclasses import replace
+
 import numpy as np
 import pytest
 import torch
@@ -250,11 +252,13 @@ def test_small_decode_step_on_library_products(gpu, shape, monkeypatch):
     test_decode_step_graph_replays_match_eager(gpu, shape)
 
 
-@pytest.mark.parametrize("tokens", [128, 129, 224, 225])
-def test_decode_step_at_the_edges_of_its_dispatch(gpu, tokens, monkeypatch):
-    """Both sides of HEAD_ROWS and linear.MAX_ROWS: which products run, and the logits against a step whose products
+@pytest.mark.parametrize("tokens,inter", [(128, 1024), (129, 1024), (224, 1024), (225, 1024), (128, 12416), (129, 12416),
+                                          (224, 12288)])
+def test_decode_step_at_the_edges_of_its_dispatch(gpu, tokens, inter, monkeypatch):
+    """Both sides of HEAD_ROWS, linear.MAX_ROWS and linear.swiglu_pays: which products run, and the logits against a step whose products
     are all the library's (bf16 roundings through four layers: the oracle test's 1% of the mean |logit|)."""
-    say("decode step dispatch", tokens)
+    say("decode step dispatch", tokens, inter)
+    shape = replace(SMALL, intermediate_size=inter)
     ql = np.full(tokens // 5, 5)
     ql[: tokens - int(ql.sum())] += 1
     ctx = 20 + (np.arange(len(ql)) * 37) % 300
@@ -265,8 +269,8 @@ def test_decode_step_at_the_edges_of_its_dispatch(gpu, tokens, monkeypatch):
     for library in (False, True):
         if library:
             monkeypatch.setattr(lin, "MAX_ROWS", 0)
-        w = DecodeWeights(SMALL, gpu, seed=9)
-        caches = alloc_kv_caches(SMALL, pool, gpu, seed=9)
+        w = DecodeWeights(shape, gpu, seed=9)
+        caches = alloc_kv_caches(shape, pool, gpu, seed=9)
         step = MixedDecodeStep(w, caches, ctx, ql, np.zeros(len(ql), bool), torch.from_numpy(table), budget=8,
                                refresh_layer=2, seed=9)
         assert step.T == tokens
@@ -278,7 +282,8 @@ def test_decode_step_at_the_edges_of_its_dispatch(gpu, tokens, monkeypatch):
         logits.append(step.logits.float().cpu())
         calls.append((count["linear"], count["partials"]))
     layers = SMALL.n_layer
-    assert calls[0] == ((layers + (tokens <= 128), 3 * layers) if tokens <= 224 else (0, 0)) and calls[1] == (0, 0)
+    own_swiglu = layers if tokens <= 128 or inter <= 12288 else 0
+    assert calls[0] == ((own_swiglu + (tokens <= 128), 3 * layers) if tokens <= 224 else (0, 0)) and calls[1] == (0, 0)
     a, b = logits
     assert (a - b).abs().mean() <= 0.01 * b.abs().mean() and (a - b).abs().max() <= 0.05 * b.abs().max()
 
