@@ -18,8 +18,8 @@ sparse_draft_runner.py:248-250). ``order="logical"`` (default) sorts by logical
 page index, identical to the reference for an increasing table and correct for
 any table; ``order="physical"`` reproduces the reference's rule literally.
 
-``KeyMeanPageSelector`` is the per-(request, KV head) selector of BASELINE
-config 2, which has no reference counterpart: page scores come from the
+``KeyMeanPageSelector`` is a selector per (request, KV head),
+which has no reference counterpart: page scores come from the
 attention kernel's key-mean epilogue (``HolisticAttentionWrapper.run(...,
 page_scores=...)``) and the top ``k`` pages per (request, kv head) are kept.
 """
@@ -213,7 +213,7 @@ class PageSelectorFirstLastAvg(PageSelector):
 
 
 class KeyMeanPageSelector:
-    """Top-k pages per (request, KV head) by the key-mean score (BASELINE config 2).
+    """Top-k pages per (request, KV head) by the key-mean score.
 
     ``page_scores`` is the ``[max_batch * H_kv, max_pages]`` fp32 buffer to pass
     to ``HolisticAttentionWrapper.run(..., page_scores=...)``; ``select`` then

@@ -8,7 +8,7 @@
 // rows, k is split over workgroups where the tiles do not fill the chip, and the fp32 partial sums go
 // to a kernel that reads the layer's output anyway (aspire_add_rms_norm_partials, the q/k preparation).
 //   * Both operands travel HBM -> LDS directly (buffer_load ... lds, full 128- or 256-byte row pieces)
-//     into rings of 4 to 7 steps of 64 or 128 k: 40-100 KB a CU in flight. Past 64 rows half of the
+//     into rings of 3 to 7 steps of 64 or 128 k: 40-100 KB a CU in flight. Past 64 rows half of the
 //     waves load w and half x, so that the w ring can be deeper than the larger x ring.
 //   * One barrier a step; a wave multiplies one set of fragments (16x16x32 MFMAs, w as the A operand:
 //     a lane's 4 results are 4 neighbouring output columns) while it reads the next.
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_kernel(LinearParams p) {
   auto at_step = [&](int s) { return s + turn < steps ? s + turn : s + turn - steps; };
   const int n0 = tile * (kOut == Out::kSwiglu ? kBN / 2 : kBN);
 
-  // ---- loads: slot L of a stage holds rows kRpi L .. of it, chunk c of row q at c ^ (q % kCh)
+  // ---- loads: slot L of a stage holds rows kRpi L .. of it, chunk c of row q at c ^ swizzle(q)
   const int lrow = lane / kCh, lpos = lane % kCh;
   const bool loads_w = !kRoles || wave < kLoadersW;
   const int lw = wave, la = kRoles ? wave - kLoadersW : wave;

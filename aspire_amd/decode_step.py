@@ -22,7 +22,7 @@ the residual adds, norms and token pick are the row kernels of the HIP library
 (``aspire_add_rms_norm``, ``aspire_argmax_rows``), so a whole step can be
 recorded in one HIP graph.
 
-Refresh layer, ``selector="keymean"`` (BASELINE config 2's selection): at
+Refresh layer, ``selector="keymean"`` (a selection per KV head): at
 ``refresh_layer`` every row attends its full context and the kernel writes the
 key-mean page scores of the single-query (draft) rows; the top-``budget`` pages
 per (row, KV head), the last ``recent_pages`` forced in, become the draft rows'
@@ -60,8 +60,10 @@ from aspire_amd.backends.page_selector import KeyMeanPageSelector, PageSelectorF
 
 PAGE = 16
 DRAFT_MODE, VERIFY_MODE = 0, 1
-# Tokens up to which the vocabulary projection runs on aspire_linear: at 151,936 x 4,096 it takes 196 us
-# at 12 rows, 210 at 48 and 249 at 104 where hipBLASLt takes 244, 262 and 277, but 355 against 324 at 208.
+# Tokens up to which the vocabulary projection runs on aspire_linear: at 151,936 x 4,096 it takes 191 us
+# at 12 rows, 200 at 48, 251 at 104 and 266 at 128 where hipBLASLt takes 258, 260, 289 and 295, but 355 against 324 at
+# 208 (past 128 rows its tiles are 64 or 96 weight rows). At widths of 2,048 and 5,120 and vocabularies of 32,000 and
+# 128,256 it is 0 to 53% shorter up to 128 rows, too; at a width of 1,024 past 64 rows 0 to 8% longer.
 HEAD_ROWS = 128
 
 

@@ -1,6 +1,6 @@
 """Seeded synthetic inputs for one mixed draft/verify attention layer.
 
-Shapes follow BASELINE.json's configs (page size 16, head_dim 128, bf16):
+The benchmark's workloads, by number (page size 16, head_dim 128, bf16):
 
 * config 0 - Qwen3-1.7B shape (16 q / 8 kv heads), batch 4, every context 4096
   tokens, a 1024-page pool in random-permutation order; rows 0-1 draft

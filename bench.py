@@ -4,7 +4,7 @@
 
 A step is one pass of the hot path over one batch resident in HBM: the paged
 KV append of the batch's new tokens followed by mixed draft/verify attention
-(including the split-KV merge). Default workload: BASELINE config 1, the
+(including the split-KV merge). Default workload: number 1, the
 Qwen3-8B-shape layer (32 q / 8 kv heads, head_dim 128, bf16, 16-token pages),
 batch 32 x 32768-token contexts, 16 drafting rows (q_len 1 over 128 selected
 pages) and 16 verifying rows (q_len 4, causal, full cache). ``--config 2`` runs
@@ -687,7 +687,7 @@ def measure_components(step, w, out, steps, plan_us):
         flops = 4 * 128 * 32 * keys
         pre[name] = {"us": round(us, 1), "tflops": round(flops / (us * 1e-6) / 1e12, 1),
                      "frac_of_bf16_mfma_peak": round(flops / (us * 1e-6) / 2.5e15, 4),
-                     "kernel": "prefill_kernel (aspire_prefill_run)",
+                     "kernel": "prefill_kernel (aspire_prefill_run_units)",
                      "decode_kernel_us": round(times["decode"], 1)}
         del st, po
     res["prefill"] = pre

@@ -98,7 +98,7 @@ int aspire_build_mixed_page_list(const void* mode_flags, int32_t mode_flags_elem
                                  void* stream);
 
 /* Per-(row, kv head) page lists: the consumer of the key-mean (B) selection,
- * which has no reference code (the BASELINE config-2 refresh layer feeding the
+ * which has no reference code (a refresh layer's per-head selection feeding the
  * following sparse layers). Segment s = b * num_kv_heads + g takes
  * selected_counts[s] entries of row s of `selected` ([batch * num_kv_heads,
  * selected_width], the KeyMeanPageSelector output) when row b drafts, and
@@ -191,7 +191,7 @@ int aspire_plan_upload(const aspire_plan_layout* layout, const aspire_plan_info*
  * 257-273) and, when dump_kind != 0, the logits-dump variant bound at the
  * refresh layer (aspire/backends/base.py:452-514, jit_kernels.py:74-96,
  * 182-193, 247-256). page_scores != NULL adds the per-KV-head key-mean page
- * score of BASELINE config 2 (no reference counterpart). */
+ * score of the per-head selection (no reference counterpart). */
 typedef struct aspire_attention_args {
   const void* q; int64_t q_stride_t; int64_t q_stride_h;
   const void* kv_cache; int64_t cache_stride_p; int64_t cache_stride_kv;
@@ -424,7 +424,7 @@ int aspire_rope_frequencies(int32_t head_dim, float rope_theta, float rope_scale
 
 /* ------------------------------------------------ decode-step row operations
  * The per-token steps a decode step runs between the GEMMs, used by the full
- * decode step (BASELINE config 3). One workgroup per row, no scratch memory.
+ * decode step. One workgroup per row, no scratch memory.
  *
  * aspire_add_rms_norm: with delta, x[r] += delta[r] (bf16) first
  * (h = x + attn_out, aspire/models/sparse_draft_transformer.py:232-238); then
@@ -449,7 +449,8 @@ int aspire_linear(const void* x, int64_t x_stride, const void* w, int64_t w_stri
                   int64_t out_stride, int32_t rows, int32_t n, int32_t k, int32_t swiglu, void* stream);
 
 /* The same layer with k split: partials [splits][rows][n] fp32, whose sum over the slabs is the output,
- * for a consumer that reads it once (aspire_add_rms_norm_partials, aspire_rope_args.partials).
+ * for a consumer that reads it once (aspire_add_rms_norm_partials,
+ * aspire_qk_norm_rope_append_partials).
  * aspire_linear_splits says how many slabs a shape takes (0: refused; host only). */
 int32_t aspire_linear_splits(int32_t rows, int32_t n, int32_t k);
 int aspire_linear_partials(const void* x, int64_t x_stride, const void* w, int64_t w_stride, float* partials,
@@ -495,6 +496,7 @@ typedef struct aspire_prefill_args {
  * group does not divide a wave's query rows (32 in the default build). Host only. */
 int aspire_prefill_block_tokens(int32_t num_qo_heads, int32_t num_kv_heads);
 
+/* Every query block whole, the last one first. */
 int aspire_prefill_run(const aspire_prefill_args* args, void* stream);
 
 /* The same with the blocks' keys cut into pieces, for batches whose blocks are too few or too uneven to

@@ -22,7 +22,7 @@ running FlashInfer's persistent kernel, patched by
   query ``qo_len-1`` to its single slot. The dump is taken before the causal
   mask, so masked keys are still dumped. Only ``j < kv_len`` is written.
 
-The per-KV-head page-score epilogue (BASELINE config 2) has no reference
+The per-KV-head page-score epilogue has no reference
 counterpart: for a ``qo_len == 1`` row, page ``j`` of kv head ``g`` scores
 ``max_{h in group(g)} q_h . mean_t(k_{j,t,g})`` over the page's valid keys.
 

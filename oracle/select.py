@@ -21,7 +21,7 @@
     index instead and gives the identical result for an increasing table;
     ``order="physical"`` is the reference's literal rule.
 
-(B) The per-(request, KV head) key-mean selector of BASELINE config 2, which
+(B) The per-(request, KV head) key-mean selector, which
     has no reference counterpart: page ``j`` of kv head ``g`` scores
     ``max_{h in group(g)} q_h . mean_t(k_{j,t,g})`` (``oracle.attention``'s
     page-score epilogue); the top ``k`` pages per (request, kv head) are kept,

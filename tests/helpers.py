@@ -21,7 +21,7 @@ def bits(t: torch.Tensor) -> np.ndarray:
 
 
 def attn_close(out: torch.Tensor, ref: torch.Tensor, max_abs=2e-2, mean_abs=2e-3):
-    """BASELINE tolerance for bf16 attention output with fp32 accumulation."""
+    """The tolerance for bf16 attention output with fp32 accumulation."""
     d = (out.float().cpu() - ref.float().cpu()).abs()
     assert torch.isfinite(out.float()).all(), "non-finite output"
     assert d.max().item() <= max_abs, f"max abs {d.max().item():.4g} > {max_abs}"

@@ -1,4 +1,4 @@
-"""BASELINE config 3 at its real workload: the full 36-layer Qwen3-8B decode step, batch 64,
+"""Workload 3 at its real size: the full 36-layer Qwen3-8B decode step, batch 64,
 contexts U[8192, 32768], a 50/50 draft/verify mix with verify q_len U{2..9}, refresh at layer 2
 with the top-128 pages per (row, KV head).
 

@@ -1,10 +1,10 @@
-"""BASELINE configs 2 and 4 at their real workloads, the (R) selector at refresh-layer scale,
+"""Workloads 2 and 4 at their real sizes, the (R) selector at refresh-layer scale,
 and masking of stale cache slots past each row's length, on the GPU against the CPU oracle.
 
-Config 2 (workloads.config2): the B=64 refresh layer, contexts
+Workload 2 (workloads.config2): the B=64 refresh layer, contexts
 U[8192, 32768], full attention for 64 single-query rows with the per-KV-head key-mean page
-scores, top-128 pages per (row, kv head). Config 4 (workloads.config4, configs[4]): batch 16
-over 64k-128k contexts at every draft fraction the config sweeps. Sampled rows are checked
+scores, top-128 pages per (row, kv head). Workload 4 (workloads.config4): batch 16
+over 64k-128k contexts at every draft fraction the workload sweeps. Sampled rows are checked
 against the oracle after their pages are gathered on the device; properties that need no
 oracle (finite output, the exact top-k of the GPU's own scores) are checked on every row.
 """
